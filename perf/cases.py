@@ -305,7 +305,7 @@ def prepare(case, seed):
         state["boundary"] = [sim.boundary(0, d) for d in (0, 1)]
     if call == "newton":
         # all Krylov directions of one cycle
-        sim.set_newton_options(restarts=1, eta_max=1e-6)
+        sim.set_newton_options(restarts=1, eta_max=1e-4)
     return state
 
 
