@@ -73,7 +73,7 @@ __device__ __forceinline__ Cx<double> stepAdjoint(const StepSite<double> &p, dou
                                                   Cx<double> y0, Cx<double> y, Cx<double> ybar,
                                                   double hs, Cx<double> &dbar, double &ebar) {
   const Cx<double> w = y + y0;
-  const Cx<double> aw = p.a * w;
+  const Cx<double> aw = p.a() * w;
   const Cx<double> fy = {2.0 * aw.re + ser - 1.0, 2.0 * aw.im + p.sei};
   const Cx<double> fy0 = {2.0 * aw.re + ser + 1.0, 2.0 * aw.im + p.sei};
   const double r = rcpT(fy.re * fy.re + fy.im * fy.im);
@@ -830,12 +830,12 @@ __device__ __forceinline__ Cx<double> stepTangent(const StepSite<double> &p,
                                                   const StepSite<double> &pt, double ser,
                                                   Cx<double> y0, Cx<double> y, Cx<double> dy0) {
   const Cx<double> w = y + y0;
-  const Cx<double> aw = p.a * w;
+  const Cx<double> aw = p.a() * w;
   const Cx<double> fy = {2.0 * aw.re + ser - 1.0, 2.0 * aw.im + p.sei};
   const Cx<double> fy0 = {2.0 * aw.re + ser + 1.0, 2.0 * aw.im + p.sei};
   const double r = rcpT(fy.re * fy.re + fy.im * fy.im);
   const Cx<double> q = {-fy.re * r, fy.im * r};
-  const Cx<double> dF = fy0 * dy0 + (w * w) * pt.a + pt.sD + Cx<double>{-w.im * pt.sei, w.re * pt.sei};
+  const Cx<double> dF = fy0 * dy0 + (w * w) * pt.a() + pt.sD() + Cx<double>{-w.im * pt.sei, w.re * pt.sei};
   return q * dF;
 }
 
@@ -1226,7 +1226,7 @@ void Grain::prepareAdjoint() {
     std::vector<SweepItem> items = sweepItems(s, gv.cols, &adjMaxLen_);
     std::vector<SweepItemDev> di(items.size());
     for (size_t i = 0; i < items.size(); ++i)
-      di[i] = {0, items[i].angle, items[i].x0, items[i].ncols, items[i].ylo, items[i].yhi};
+      di[i] = {0, items[i].angle, items[i].x0, items[i].ncols, items[i].ylo, items[i].yhi, items[i].reentered};
     adjNumItems_ = static_cast<int>(di.size());
     SC_HIP(hipMalloc(&adjItems_, std::max<size_t>(1, di.size()) * sizeof(SweepItemDev)));
     if (!di.empty()) toDevice(adjItems_, di.data(), di.size() * sizeof(SweepItemDev));

@@ -39,6 +39,8 @@ template <typename T> __device__ __forceinline__ GlobalPtr<T> global(T *p) {
   return (GlobalPtr<T>)p;
 }
 
+template <typename T> using LdsPtr = __attribute__((address_space(3))) T *;
+
 // Streaming access to the sweep scratch: every element is written once and
 // read once, so the accesses carry the non-temporal hint and leave the cache
 // to the grids the sweep samples.
@@ -58,55 +60,76 @@ template <typename T> __device__ __forceinline__ Cx<T> loadStream(const Cx<T> *p
   return Cx<T>{w.x, w.y};
 }
 
-// Reciprocal and reciprocal square root.  FP32: the hardware v_rcp_f32 /
-// v_rsq_f32 (1 ulp).  FP64: the hardware v_rcp_f64 / v_rsq_f64 estimate
-// refined by kNewtonSteps Newton-Raphson iterations (each doubles the number
-// of correct bits of the roughly single-precision estimate; two reach the
-// last bits of the double), instead of the longer IEEE division and square
-// root sequences.
-constexpr int kNewtonSteps = 2;
+// Reciprocal, reciprocal square root and square root.  FP32: the hardware
+// v_rcp_f32 / v_rsq_f32 (1 ulp).  FP64: the hardware v_rcp_f64 / v_rsq_f64
+// estimate (largest relative error measured over 2^-6 to 2^6: 4.6e-8 and
+// 5.3e-8) refined by one third-order step, whose error is of the order of the
+// cube of the estimate's (1e-22): 3 and 5 instructions to the last bits
+// (1.1e-16 and 1.4e-16 measured), against 4 and 7 for two Newton steps.
+__device__ __forceinline__ float fmaT(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fmaT(double a, double b, double c) { return fma(a, b, c); }
 __device__ __forceinline__ float rcpT(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ float rsqT(float x) { return __builtin_amdgcn_rsqf(x); }
+__device__ __forceinline__ float sqrtT(float x) { return x * __builtin_amdgcn_rsqf(x); }
 __device__ __forceinline__ double rcpT(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-#pragma unroll
-  for (int i = 0; i < kNewtonSteps; ++i) r = fma(r, fma(-x, r, 1.0), r);
-  return r;
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r); // r (1 + e + e^2)
 }
 __device__ __forceinline__ double rsqT(double x) {
-  // r += r (1 - x r^2) / 2, with the halving applied to x once: scaling by
-  // 0.5 is exact, so this is the same arithmetic one multiply shorter
-  const double hx = 0.5 * x;
-  double r = __builtin_amdgcn_rsq(x);
-#pragma unroll
-  for (int i = 0; i < kNewtonSteps; ++i) {
-    const double he = fma(-(hx * r), r, 0.5); // (1 - x r^2) / 2
-    r = fma(r, he, r);
-  }
-  return r;
+  const double r = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * r), r, 1.0);
+  return fma(r * e, fma(e, 0.375, 0.5), r); // r (1 + e/2 + 3 e^2 / 8)
+}
+// sqrt(x) of a positive x: the step of rsqT applied to x r
+__device__ __forceinline__ double sqrtT(double x) {
+  const double r = __builtin_amdgcn_rsq(x);
+  const double g = x * r;
+  const double e = fma(-g, r, 1.0);
+  return fma(g * e, fma(e, 0.375, 0.5), g);
 }
 // Kept for the host-visible unit checks and the bulk solution.
 __device__ __forceinline__ double drcp(double x) { return rcpT(x); }
 __device__ __forceinline__ float drcp(float x) { return rcpT(x); }
 
-// Principal complex square root (Kahan's formulation): with
-// t = sqrt((|x| + |z|) / 2), sqrt(z) = (t, y / 2t) for x >= 0 and
-// (|y| / 2t, copysign(t, y)) otherwise.  Both square roots come from
-// reciprocal square roots: |z| = n rsq(n) with n = |z|^2, and with
-// u = (|x| + |z|) / 2, t = u rsq(u) and y / 2t = y rsq(u) / 2.
-// n is held at or above the smallest normal number, so z = 0 gives a root
-// of order 1e-77 (1e-10 in FP32) instead of 0 -- negligible beside the O(1)
-// terms it is added to -- with no branch and no select: the square roots of
-// a lane's energies stay in one basic block and their latencies overlap.
-template <typename T> __device__ __forceinline__ Cx<T> csqrt(Cx<T> z) {
-  const T n = fmax(z.re * z.re + z.im * z.im, std::numeric_limits<T>::min());
-  const T m = n * rsqT(n);
-  const T u = T(0.5) * (fabs(z.re) + m);
+// sqrt(2) times the principal complex square root (Kahan's formulation): with
+// u = |x| + |z|, sqrt(2 z) = (sqrt(u), y / sqrt(u)) for x >= 0 and
+// (|y| / sqrt(u), copysign(sqrt(u), y)) otherwise; both parts come from one
+// reciprocal square root of u.
+// |z|^2 is held at or above the smallest normal number, so z = 0 gives a
+// root of order 1e-77 (1e-10 in FP32) instead of 0 -- negligible beside the
+// O(1) terms it is added to -- with no branch and no select: the square roots
+// of a lane's energies stay in one basic block and their latencies overlap.
+template <typename T> __device__ __forceinline__ Cx<T> csqrt2(Cx<T> z) {
+#pragma clang fp contract(off)
+  const T n = fmaT(z.re, z.re, fmaT(z.im, z.im, std::numeric_limits<T>::min()));
+  const T u = fabs(z.re) + sqrtT(n);
   const T r = rsqT(u);
   const T t = u * r;
-  const T q = (T(0.5) * z.im) * r;
+  const T q = z.im * r;
   const bool right = z.re >= T(0);
   return {right ? t : fabs(q), right ? q : copysign(t, z.im)};
+}
+template <typename T> __device__ __forceinline__ Cx<T> csqrt(Cx<T> z) {
+  return scale(csqrt2(z), T(0.70710678118654752440));
+}
+
+// The sign of every x seen so far: negative once one was.
+__device__ __forceinline__ void noteSign(int &neg, float x) { neg |= __float_as_int(x); }
+__device__ __forceinline__ void noteSign(int &neg, double x) { neg |= __double2hiint(x); }
+
+// The root of a step's discriminant.  WHOLE: of any z.  Else of z with
+// z.re >= 0, two multiplies without the 7 instructions of the selects, and neg
+// turns negative where that does not hold: the caller takes the steps again.
+template <bool WHOLE, typename T>
+__device__ __forceinline__ Cx<T> stepRoot2(Cx<T> z, int &neg) {
+#pragma clang fp contract(off)
+  if constexpr (WHOLE) return csqrt2(z);
+  noteSign(neg, z.re);
+  const T n = fmaT(z.re, z.re, fmaT(z.im, z.im, std::numeric_limits<T>::min()));
+  const T u = z.re + sqrtT(n);
+  const T r = rsqT(u);
+  return {u * r, z.im * r};
 }
 
 // a / b through the reciprocal of |b|^2 (|b| is of order one here).
@@ -115,39 +138,133 @@ template <typename T> __device__ __forceinline__ Cx<T> cdiv(Cx<T> a, Cx<T> b) {
   return {(a.re * b.re + a.im * b.im) * r, (a.im * b.re - a.re * b.im) * r};
 }
 
-// One implicit-midpoint step of the Riccati equation solved as the quadratic
-// a y^2 + b y + c = 0 (RiccatiSolutions.h:65-94):
-//   s = i h, a = s conj(D) / 4, b = 2 a y0 + s e - 1,
-//   c = (a y0 + s e + 1) y0 + s D,  y = 2 c / (-b + sqrt(b^2 - 4 a c)).
+// One implicit-midpoint step of the Riccati equation (RiccatiSolutions.h:65-94):
+// y solves a (y + y0)^2 + (s e - 1) y + (s e + 1) y0 + s D = 0 with s = i h and
+// a = s conj(D) / 4; with disc = (s e - 1)^2 + h^2 |D|^2 - 8 a y0, where only the
+// last term depends on y0, and R = sqrt(disc),
+//   y = y0 + 2 (y0 w + s D) / (2 - w),   w = s e + 1 - R            (FP64)
+//   y = y0 + 4 C / (R - B),   B = s e - 1 + 2 alpha,  alpha = 2 a y0,
+//                             C = (alpha + s e) y0 + s D / 2       (FP32).
+// The two are the same root, solved for the increment of y: the FP32 form
+// rounds nothing that is larger than the increment (over 600 steps of h = 0.05
+// its error against FP64 is 1e-7 of y, that of the root y taken whole 2e-6);
+// the FP64 form takes 1 - R, exact in floating point, for 6 instructions less,
+// and its error is that of the root y taken whole (1e-15 of y) or below.  A step
+// is 42 (FP64) and 32 (FP32) add/multiply instructions, 3 square roots and
+// reciprocals; the root taken whole was 63.
 // The quantities that only depend on the site (D, the energy shift Re e and
 // h) are formed once per site and shared by every Ozaki energy.
-template <typename T> struct StepSite {
-  Cx<T> a;  // s conj(D) / 4
-  Cx<T> a4; // 4 a
-  Cx<T> sD; // s D = (-4 a.re, 4 a.im)
-  T sei;    // Im(s e) = h Re e
+// The arithmetic is written with explicit fused multiply-adds, so that every
+// place that takes the same step (a sweep, a segment integrated again from a
+// checkpoint, the adjoint) rounds alike.
+template <typename T> struct StepSite;
+
+// FP64: everything but w is scaled so that the quotient needs no factor, disc
+// by 1/2.
+template <> struct StepSite<double> {
+  Cx<double> a4; // 4 a = i h conj(D); s D = (-a4.re, a4.im)
+  double sei;    // Im(s e) = h Re e
+  double seir;   // sqrt(2) sei
+  double kh;     // (h^2 |D|^2 - sei^2) / 2
+  double root;   // sqrt(1/2)
+  __device__ __forceinline__ Cx<double> a() const { return {0.25 * a4.re, 0.25 * a4.im}; }
+  __device__ __forceinline__ Cx<double> sD() const { return {-a4.re, a4.im}; }
 };
-template <typename T>
-__device__ __forceinline__ StepSite<T> stepSite(Cx<T> D, T shift, T h) {
-  StepSite<T> p;
+__device__ __forceinline__ StepSite<double> stepSite(Cx<double> D, double shift, double h) {
+#pragma clang fp contract(off)
+  StepSite<double> p;
   p.a4 = {h * D.im, h * D.re};
-  p.a = {T(0.25) * p.a4.re, T(0.25) * p.a4.im};
-  p.sD = {-p.a4.re, p.a4.im};
   p.sei = h * shift;
+  p.seir = 1.41421356237309504880 * p.sei;
+  p.kh = 0.5 * fma(p.a4.re, p.a4.re, fma(p.a4.im, p.a4.im, -(p.sei * p.sei)));
+  p.root = 0.70710678118654752440;
   return p;
 }
 // ser = Re(s e) = -h Im e (the Matsubara part).
+template <bool WHOLE>
+__device__ __forceinline__ Cx<double> stepEnergy(const StepSite<double> &p, double ser,
+                                                 Cx<double> y0, int &neg) {
+#pragma clang fp contract(off)
+  const double b = fma(p.root, ser, -p.root); // (Re(s e) - 1) / sqrt(2)
+  const Cx<double> z = {fma(p.a4.im, y0.im, fma(-p.a4.re, y0.re, fma(b, b, p.kh))),
+                        fma(-p.a4.im, y0.re, fma(-p.a4.re, y0.im, p.seir * b))};
+  const Cx<double> R = stepRoot2<WHOLE>(z, neg);
+  const Cx<double> w = {(1.0 - R.re) + ser, p.sei - R.im};
+  const Cx<double> c = {fma(w.re, y0.re, fma(-w.im, y0.im, -p.a4.re)),
+                        fma(w.re, y0.im, fma(w.im, y0.re, p.a4.im))};
+  const Cx<double> q = {fma(-0.5, w.re, 1.0), 0.5 * w.im}; // conj(1 - w / 2)
+  const double r = rcpT(fma(q.re, q.re, q.im * q.im));
+  return {fma(fma(c.re, q.re, -(c.im * q.im)), r, y0.re),
+          fma(fma(c.im, q.re, c.re * q.im), r, y0.im)};
+}
+
+// FP32: scaled so that the quotient needs no factor, disc by 1/16, R - B by 1/4.
+template <> struct StepSite<float> {
+  Cx<float> a2; // 2 a = i h conj(D) / 2; s D / 2 = (-a2.re, a2.im)
+  float sei;    // Im(s e) = h Re e
+  float sei4;   // sei / 4
+  float k16;    // (h^2 |D|^2 - sei^2) / 16
+  float quarter;
+};
+__device__ __forceinline__ StepSite<float> stepSite(Cx<float> D, float shift, float h) {
+#pragma clang fp contract(off)
+  StepSite<float> p;
+  const float hh = 0.5f * h;
+  p.a2 = {hh * D.im, hh * D.re};
+  p.sei = h * shift;
+  p.sei4 = 0.25f * p.sei;
+  p.k16 = fmaf(0.25f, fmaf(p.a2.re, p.a2.re, p.a2.im * p.a2.im), -(p.sei4 * p.sei4));
+  p.quarter = 0.25f;
+  return p;
+}
+template <bool WHOLE>
+__device__ __forceinline__ Cx<float> stepEnergy(const StepSite<float> &p, float ser, Cx<float> y0,
+                                                int &neg) {
+#pragma clang fp contract(off)
+  const Cx<float> al = {fmaf(p.a2.re, y0.re, -(p.a2.im * y0.im)),
+                        fmaf(p.a2.re, y0.im, p.a2.im * y0.re)};
+  const Cx<float> v = {al.re + ser, al.im + p.sei};
+  const Cx<float> c = {fmaf(v.re, y0.re, fmaf(-v.im, y0.im, -p.a2.re)),
+                       fmaf(v.re, y0.im, fmaf(v.im, y0.re, p.a2.im))};
+  const float b = fmaf(p.quarter, ser, -p.quarter); // (Re(s e) - 1) / 4
+  const Cx<float> z = {fmaf(-p.quarter, al.re, fmaf(b, b, p.k16)),
+                       fmaf(-p.quarter, al.im, (2.f * p.sei4) * b)};
+  const Cx<float> R = stepRoot2<WHOLE>(z, neg); // sqrt(2 disc) / 4
+  constexpr float kHalfRoot = 0.70710678118654752440f;
+  const Cx<float> q = {fmaf(kHalfRoot, R.re, -fmaf(0.5f, al.re, b)),
+                       fmaf(kHalfRoot, R.im, -fmaf(0.5f, al.im, p.sei4))};
+  const float r = rcpT(fmaf(q.re, q.re, q.im * q.im));
+  return {fmaf(fmaf(c.re, q.re, c.im * q.im), r, y0.re),
+          fmaf(fmaf(c.im, q.re, -(c.re * q.im)), r, y0.im)};
+}
+
+// Real-frequency energies eps = E + i delta: sej = h E joins the site's
+// Im(s e) (the Doppler shift enters the same way).
+template <bool WHOLE>
+__device__ __forceinline__ Cx<double> stepEnergy(const StepSite<double> &p, double ser, double sej,
+                                                 Cx<double> y0, int &neg) {
+  StepSite<double> e = p;
+  e.sei = p.sei + sej;
+  e.seir = 1.41421356237309504880 * e.sei;
+  e.kh = fma(0.5 * (p.sei - e.sei), p.sei + e.sei, p.kh);
+  return stepEnergy<WHOLE>(e, ser, y0, neg);
+}
+template <bool WHOLE>
+__device__ __forceinline__ Cx<float> stepEnergy(const StepSite<float> &p, float ser, float sej,
+                                                Cx<float> y0, int &neg) {
+  StepSite<float> e = p;
+  e.sei = p.sei + sej;
+  e.sei4 = 0.25f * e.sei;
+  e.k16 = fmaf(p.sei4 - e.sei4, p.sei4 + e.sei4, p.k16);
+  return stepEnergy<WHOLE>(e, ser, y0, neg);
+}
+// a step from any y0
 template <typename T>
 __device__ __forceinline__ Cx<T> stepEnergy(const StepSite<T> &p, T ser, Cx<T> y0) {
-  const Cx<T> ay = p.a * y0;
-  const Cx<T> b = {T(2) * ay.re + (ser - T(1)), T(2) * ay.im + p.sei};
-  const Cx<T> t = {ay.re + (ser + T(1)), ay.im + p.sei};
-  const Cx<T> c = t * y0 + p.sD;
-  const Cx<T> ac4 = p.a4 * c;
-  const Cx<T> disc = {b.re * b.re - b.im * b.im - ac4.re, T(2) * b.re * b.im - ac4.im};
-  const Cx<T> sq = csqrt(disc);
-  return cdiv(c + c, sq - b);
+  int neg = 0;
+  return stepEnergy<true>(p, ser, y0, neg);
 }
+
 // Workgroups are dispatched round robin over the eight XCDs, each with its
 // own L2.  A grid of 8 * ceil(n / 8) blocks read through this mapping gives
 // every XCD a contiguous range of the n logical blocks (spatially coherent
@@ -163,20 +280,6 @@ inline unsigned xcdGrid(long long nLogical) {
   return static_cast<unsigned>(((nLogical + kNumXcd - 1) / kNumXcd) * kNumXcd);
 }
 
-// Real-frequency energies eps = E + i delta: sej = h E joins the site's
-// Im(s e) (the Doppler shift enters the same way).
-template <typename T>
-__device__ __forceinline__ Cx<T> stepEnergy(const StepSite<T> &p, T ser, T sej, Cx<T> y0) {
-  const T sei = p.sei + sej;
-  const Cx<T> ay = p.a * y0;
-  const Cx<T> b = {T(2) * ay.re + (ser - T(1)), T(2) * ay.im + sei};
-  const Cx<T> t = {ay.re + (ser + T(1)), ay.im + sei};
-  const Cx<T> c = t * y0 + p.sD;
-  const Cx<T> ac4 = p.a4 * c;
-  const Cx<T> disc = {b.re * b.re - b.im * b.im - ac4.re, T(2) * b.re * b.im - ac4.im};
-  const Cx<T> sq = csqrt(disc);
-  return cdiv(c + c, sq - b);
-}
 template <typename T>
 __device__ __forceinline__ Cx<T> riccatiStep(Cx<T> D, Cx<T> e, Cx<T> y0, T h) {
   return stepEnergy(stepSite(D, e.re, h), -h * e.im, y0);

@@ -193,6 +193,7 @@ void Grain::upload() {
   std::vector<double> dist;
   for (const auto *v : {&s.distInG, &s.distOutG, &s.distInGt, &s.distOutGt})
     dist.insert(dist.end(), v->begin(), v->end());
+  dist.push_back(0.0); // the sweep fetches one crossing past the last
   dDist_ = devUpload(dist);
   dBcOffG_ = devUpload(s.bcG.offset);
   dBcSrcG_ = devUpload(s.bcG.src);
@@ -221,9 +222,11 @@ void Grain::upload() {
   dCurrentOld_ = devAlloc<double>(2 * n0);
   dEnergyDens_ = devAlloc<double>(n0);
   const long long neCap = s.keldysh ? s.spec.perBlock : s.Ne;
-  dBInG_ = devAlloc<double>(size_t(2 * s.nInG * neCap));
+  // in-values: the sweep fetches one crossing and up to EL - 1 energies past
+  // the last
+  dBInG_ = devAlloc<double>(size_t(2 * s.nInG * neCap) + size_t(neCap) + kMaxSweepEL);
   dBOutG_ = devAlloc<double>(size_t(2 * s.nOutG * neCap));
-  dBInGt_ = devAlloc<double>(size_t(2 * s.nInGt * neCap));
+  dBInGt_ = devAlloc<double>(size_t(2 * s.nInGt * neCap) + size_t(neCap) + kMaxSweepEL);
   dBOutGt_ = devAlloc<double>(size_t(2 * s.nOutGt * neCap));
   // Keldysh grains hold spectral weights of an angle chunk instead
   if (!s.keldysh) {
@@ -258,7 +261,7 @@ void Grain::upload() {
     dZero2_ = devAlloc<double>(2);
     SC_HIP(hipMemsetAsync(dZero2_, 0, 2 * sizeof(double), stream_));
   }
-  dCounter_ = devAlloc<int>(1);
+  growCounter(dCounter_, counterCap_, 1);
 }
 
 void Grain::uploadEnergies() {
@@ -268,14 +271,6 @@ void Grain::uploadEnergies() {
   SC_HIP(hipMemcpy(dResidue_, s.residue.data(), b, hipMemcpyHostToDevice));
   if (dEnergyRe_) SC_HIP(hipMemcpy(dEnergyRe_, s.energyRe.data(), b, hipMemcpyHostToDevice));
 }
-
-// Compiled sweep variants: (energies per lane, wavefronts per SIMD), for
-// Matsubara energies and for real-frequency (Keldysh) energies.
-#define SC_SWEEP_VARIANTS(X)                                                         \
-  X(1, 4) X(2, 4) X(3, 3) X(4, 2) X(4, 3) X(4, 4) X(5, 2) X(6, 2) X(7, 1) X(7, 2) X(7, 4)  \
-  X(8, 1) X(8, 2) X(8, 4)                                                            \
-  X(14, 1) X(14, 2) X(16, 1) X(16, 2)
-#define SC_KELDYSH_VARIANTS(X) X(2, 4) X(4, 2) X(4, 3) X(4, 4) X(8, 1) X(8, 2) X(8, 4) X(16, 1)
 
 bool sweepVariantExists(int el, int waves, bool keldysh) {
 #define SC_HAS(E, W) if (el == E && waves == W) return true;
@@ -322,6 +317,7 @@ void Grain::prepareSweep(int precision) {
   pl.cols = gv.cols;
   std::vector<SweepItem> items = sweepItems(s, pl.cols, &pl.maxLen);
   pl.numItems = static_cast<int>(items.size());
+  growCounter(dCounter_, counterCap_, pl.numItems);
   // Keldysh grains sweep by angle chunks: the items of a chunk are
   // contiguous (still longest first within it) and name the view whose
   // angle base is the chunk's first angle.
@@ -354,7 +350,7 @@ void Grain::prepareSweep(int precision) {
   std::vector<SweepItemDev> di(items.size());
   for (size_t i = 0; i < items.size(); ++i)
     di[i] = {s.keldysh ? items[i].angle / pl.chunkAngles : 0, items[i].angle, items[i].x0,
-             items[i].ncols, items[i].ylo, items[i].yhi};
+             items[i].ncols, items[i].ylo, items[i].yhi, items[i].reentered};
   if (pl.dItems) (void)hipFree(pl.dItems);
   pl.dItems = nullptr;
   SC_HIP(hipMalloc(&pl.dItems, std::max<size_t>(1, di.size()) * sizeof(SweepItemDev)));
@@ -886,30 +882,20 @@ void Grain::ensureBoundaryInit() {
   boundaryInit_ = true;
 }
 
-template <typename T, int EL, int W, bool KEL>
-static void launchSweep(const SweepArgs &a, int slots, hipStream_t st) {
-  sweepKernel<T, EL, W, KEL><<<slots, 64, 0, st>>>(a, a.views, a.items);
-}
-
 void launchSweepVariant(int precision, int el, int waves, const SweepArgs &a, int slots,
                         hipStream_t stream, bool keldysh) {
-  const bool dp = precision == PREC_FP64;
-#define SC_LAUNCH(E, W)                                                              \
-  if (el == E && waves == W) {                                                       \
-    if (dp) launchSweep<double, E, W, KEL>(a, slots, stream);                        \
-    else launchSweep<float, E, W, KEL>(a, slots, stream);                            \
-    SC_HIP(hipGetLastError());                                                       \
-    return;                                                                          \
-  }
-  if (keldysh) {
-    constexpr bool KEL = true;
-    SC_KELDYSH_VARIANTS(SC_LAUNCH)
-  } else {
-    constexpr bool KEL = false;
-    SC_SWEEP_VARIANTS(SC_LAUNCH)
-  }
-#undef SC_LAUNCH
-  throw std::runtime_error("sweep variant not compiled");
+  if (!(precision == PREC_FP64 ? launchSweepFp64 : launchSweepMixed)(el, waves, a, slots, stream,
+                                                                     keldysh))
+    throw std::runtime_error("sweep variant not compiled");
+}
+
+void growCounter(int *&counter, size_t &cap, int numItems) {
+  const size_t need = size_t(kAgainList) + size_t(std::max(numItems, 1));
+  if (need <= cap) return;
+  devFree(counter);
+  cap = 0;
+  counter = devAlloc<int>(need);
+  cap = need;
 }
 
 void Grain::sweep(int precision, bool burnin) {
@@ -2100,7 +2086,7 @@ Batch::Batch(std::vector<std::unique_ptr<Setup>> setups) {
     grains_.back()->initialGuess();
   }
   done_.assign(grains_.size(), 0);
-  dCounter_ = devAlloc<int>(1);
+  growCounter(dCounter_, counterCap_, 1);
 }
 
 Batch::~Batch() {
@@ -2185,7 +2171,7 @@ void Batch::prepare(int precision, const std::vector<int> &act) {
   for (int gi : act) {
     pl.maxLen = std::max(pl.maxLen, pl.maxLenOf[size_t(gi)]);
     for (const SweepItem &it : pl.itemsOf[size_t(gi)]) {
-      items.push_back({gi, it.angle, it.x0, it.ncols, it.ylo, it.yhi});
+      items.push_back({gi, it.angle, it.x0, it.ncols, it.ylo, it.yhi, it.reentered});
       lens.push_back(it.yhi - it.ylo + 1);
     }
   }
@@ -2213,6 +2199,7 @@ void Batch::prepare(int precision, const std::vector<int> &act) {
   pl.numFieldJobs = static_cast<int>(act.size());
   pl.numFieldTiles = tiles;
   pl.numItems = static_cast<int>(sorted.size());
+  growCounter(dCounter_, counterCap_, pl.numItems);
   if (sorted.size() > pl.itemsCap || !pl.dItems) {
     if (pl.dItems) (void)hipFree(pl.dItems);
     pl.dItems = nullptr;

@@ -14,6 +14,11 @@
 
 namespace scamd {
 
+// Room for the sweep's work counters over numItems items (no work may be
+// using them).
+void growCounter(int *&counter, size_t &cap, int numItems);
+
+
 enum Precision { PREC_FP64 = 0, PREC_MIXED = 1, PREC_MIXED_REFINE = 2 };
 // Newton-Krylov's exact Jacobian-vector products (the tangent-linear sweep)
 constexpr int JVP_TANGENT = 3;
@@ -455,7 +460,8 @@ private:
   SweepPlan plan_[2];
   void *dScratch_ = nullptr;
   size_t scratchBytes_ = 0;
-  int *dCounter_ = nullptr;
+  int *dCounter_ = nullptr; // the sweep's work counters (sc_view.hpp)
+  size_t counterCap_ = 0;
   // accelerator state (history lives on the device)
   int accIter_ = 0;
   std::vector<double *> accX_, accD_;
@@ -616,7 +622,8 @@ private:
   Plan plan_[2];
   void *dScratch_ = nullptr;
   size_t scratchBytes_ = 0;
-  int *dCounter_ = nullptr;
+  int *dCounter_ = nullptr; // the sweep's work counters (sc_view.hpp)
+  size_t counterCap_ = 0;
   // start and end of the last sweep launch per precision; the iteration
   hipEvent_t ev0_[2] = {nullptr, nullptr}, ev1_[2] = {nullptr, nullptr};
   hipEvent_t evIt0_ = nullptr, evIt1_ = nullptr;
@@ -626,6 +633,10 @@ private:
 
 // One launch of the compiled sweep variant (precision, energies per lane,
 // wavefronts per SIMD) over the items of `args`.
+bool launchSweepFp64(int el, int waves, const SweepArgs &args, int slots, hipStream_t stream,
+                     bool keldysh);
+bool launchSweepMixed(int el, int waves, const SweepArgs &args, int slots, hipStream_t stream,
+                      bool keldysh);
 void launchSweepVariant(int precision, int el, int waves, const SweepArgs &args, int slots,
                         hipStream_t stream, bool keldysh = false);
 bool sweepVariantExists(int el, int waves, bool keldysh = false);

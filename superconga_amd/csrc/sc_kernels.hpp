@@ -60,7 +60,12 @@ __device__ __forceinline__ void siteFields(const GrainView &v, int k, int x,
   }
 }
 
-__global__ void resetCounter(int *c) { *c = 0; }
+// The sweep's work counters (sc_view.hpp).
+__global__ void resetCounter(int *c) {
+  c[0] = 0;
+  c[1] = 0;
+  c[kAgainCount] = 0;
+}
 
 // The site fields a sweep reads, for the tiles of frames [k0, ...): each
 // block covers one tile (16 adjacent columns of one frame and the rows a
@@ -109,397 +114,6 @@ __global__ void fieldsBatchKernel(const GrainView *__restrict__ views,
   // by the sweep that follows
   fieldsTile(v, v.fieldTiles + 4 * (b - tileStart[lo]), 0, v.fieldPlane,
              const_cast<double *>(v.fields));
-}
-
-// One step for one energy: Matsubara energies (i omega) or, with KEL,
-// real-frequency energies E + i delta.
-template <bool KEL, typename T>
-__device__ __forceinline__ Cx<T> stepE(const StepSite<T> &p, T ser, T sej, Cx<T> y0) {
-  if constexpr (KEL) return stepEnergy(p, ser, sej, y0);
-  else return stepEnergy(p, ser, y0);
-}
-
-// The Riccati sweep.  One wavefront handles an item: `cols` adjacent columns
-// of one frame; each column is carried by `groups` lanes holding EL Ozaki
-// energies each (lane = group * cols + column; the 64 - groups * cols lanes
-// past the last group idle).  Pass 1 integrates gamma~ from the top of the
-// item to the bottom and keeps it in the slot's scratch; pass 2 integrates
-// gamma upwards and forms the energy-summed Green functions at every inside
-// site.  Boundary in-values are read and out-values written as in
-// RiccatiSolverConfined.h:129-312.
-//
-// The order parameter and Doppler shift of a row are computed once per
-// column: the lanes of a column take consecutive rows of a chunk and pass
-// the values round with __shfl.
-template <typename T, int EL, bool KEL>
-__device__ __forceinline__ void sweepItem(const SweepArgs &a, const GrainView &v,
-                                          const SweepItemDev &it, Cx<T> *scr) {
-  const int lane = threadIdx.x;
-  const int cols = v.cols;
-  const int gp = v.groups; // lanes per column
-  const int g = lane / cols;
-  const int c = lane - g * cols;
-  const int N1 = v.N1, Ne = v.Ne;
-  const size_t n1 = size_t(N1) * N1;
-  const T h = T(v.h);
-  const int k = it.angle;
-  const bool colActive = c < it.ncols;
-  const int x = it.x0 + (colActive ? c : it.ncols - 1);
-  const bool active = colActive && (g < v.groups);
-  const GlobalPtr<const int8_t> lab = global(v.labels + size_t(k) * n1 + x);
-  T ser[EL], sej[EL], res[EL];
-  bool eOk[EL];
-#pragma unroll
-  for (int j = 0; j < EL; ++j) {
-    const int e = g * EL + j;
-    eOk[j] = active && e < Ne;
-    ser[j] = eOk[j] ? -h * T(global(v.energy)[e]) : T(0);
-    sej[j] = (KEL && eOk[j]) ? h * T(global(v.energyRe)[e]) : T(0);
-    res[j] = eOk[j] ? T(global(v.residue)[e]) : T(0);
-  }
-  const int len = it.yhi - it.ylo + 1;
-  const size_t col = size_t(k) * N1 + x;
-
-  // ---------------- pass 1: gamma~ along -y ----------------
-  {
-    const int baseIn = global(v.idxInGt)[col], baseOut = global(v.idxOutGt)[col];
-    int cntIn = 0, cntOut = 0;
-    Cx<T> coh[EL];
-#pragma unroll
-    for (int j = 0; j < EL; ++j) coh[j] = {T(0), T(0)};
-    Cx<T> dPrev = {T(0), T(0)};
-    T esPrev = T(0);
-    bool havePrev = false;
-    int8_t lcur = lab[size_t(it.yhi) * N1];
-    // the fields and label of the lane's row of the next chunk, loaded while
-    // the current chunk is swept
-    double nre = 0.0, nim = 0.0, nes = 0.0;
-    int nlab = 0;
-    auto loadChunk = [&](int t0) {
-      const int tt = t0 + g;
-      if (colActive && g < gp && tt < len) {
-        const int y = it.yhi - tt;
-        const size_t fi = size_t(k - v.fieldBase) * n1 + size_t(y) * N1 + x;
-        nre = global(v.fields)[fi];
-        nim = global(v.fields)[v.fieldPlane + fi];
-        nes = global(v.fields)[2 * v.fieldPlane + fi];
-        nlab = lab[size_t(y) * N1];
-      } else {
-        nre = nim = nes = 0.0;
-        nlab = 0;
-      }
-    };
-    loadChunk(0);
-    for (int t0 = 0; t0 < len; t0 += gp) {
-      const double fre = nre, fim = nim, fes = nes;
-      const int flab = nlab;
-      const bool more = t0 + gp < len;
-      if (more) loadChunk(t0 + gp);
-      // at least one site (t0 < len, gp >= 1): with no zero-trip path every
-      // way to the next chunk passes a site's memory operations, and the
-      // wait for this chunk's loads there is counted past them
-      const int tEnd = max(1, min(gp, len - t0));
-      for (int i = 0; i < tEnd; ++i) {
-        const int src = i * cols + c;
-        const double dre = __shfl(fre, src), dim = __shfl(fim, src), e = __shfl(fes, src);
-        const int t = t0 + i;
-        // the next site's label: in this chunk, or the first row of the next
-        const int ln = i + 1 < tEnd ? __shfl(flab, src + cols) : (more ? __shfl(nlab, c) : 0);
-        const int8_t lnext = int8_t(ln);
-        const Cx<T> D = {T(-dre), T(dim)}; // -conj(Delta) for gamma~
-        const T es = T(e);
-        if (active) {
-          if (lcur == 1 || lcur == 2) {
-            // inside (1) or exit of gamma~ (2): midpoint step
-            const Cx<T> Dm = {(dPrev.re + D.re) * T(0.5), (dPrev.im + D.im) * T(0.5)};
-            const StepSite<T> ps = stepSite(Dm, (esPrev + es) * T(0.5), h);
-            const T half = havePrev ? T(1) : T(0.5);
-#pragma unroll
-            for (int j = 0; j < EL; ++j) coh[j] = stepE<KEL>(ps, ser[j] * half, sej[j] * half, coh[j]);
-            if (lcur == 2) {
-              const int ci = baseOut + cntOut;
-              const T dr = T(global(v.distOutGt)[ci]), d = dr * h;
-              const StepSite<T> pe = stepSite(D, es, d);
-#pragma unroll
-              for (int j = 0; j < EL; ++j) {
-                if (!eOk[j]) continue;
-                const Cx<T> bv = stepE<KEL>(pe, ser[j] * dr, sej[j] * dr, coh[j]);
-                const size_t si = size_t(ci) * Ne + g * EL + j;
-                global(v.bOutGt)[si] = double(bv.re);
-                global(v.bOutGt)[size_t(v.nOutGt) * Ne + si] = double(bv.im);
-              }
-              ++cntOut;
-            }
-          } else if (lcur == 3) {
-            // entry of gamma~: start from the boundary value
-            const int ci = baseIn + cntIn;
-            const T dr = T(global(v.distInGt)[ci]), d = dr * h;
-            const StepSite<T> pe = stepSite(D, es, d);
-#pragma unroll
-            for (int j = 0; j < EL; ++j) {
-              const size_t si = size_t(ci) * Ne + g * EL + j;
-              const GlobalPtr<const double> bin = global(v.bInGt);
-              const Cx<T> b0 = eOk[j] ? Cx<T>{T(bin[si]), T(bin[size_t(v.nInGt) * Ne + si])}
-                                      : Cx<T>{T(0), T(0)};
-              coh[j] = stepE<KEL>(pe, ser[j] * dr, sej[j] * dr, b0);
-            }
-            ++cntIn;
-          } else {
-#pragma unroll
-            for (int j = 0; j < EL; ++j) coh[j] = {T(0), T(0)};
-          }
-        }
-        // gamma~ into the slot's scratch on every path through a site (the
-        // second pass reads it only where it is inside and not burning in):
-        // the wait for the next chunk's loads is then counted past these
-        // stores.  A burn-in sweep reads none, and all its lanes store into
-        // one element.
-        {
-          const size_t at = a.burnin ? 0 : size_t(t) * EL;
-          const int ln = a.burnin ? 0 : lane;
-#pragma unroll
-          for (int j = 0; j < EL; ++j)
-            storeStream(scr + (at + (a.burnin ? 0 : j)) * 64 + ln, coh[j]);
-        }
-        dPrev = D;
-        esPrev = es;
-        havePrev = true;
-        lcur = lnext;
-      }
-    }
-  }
-
-  // ---------------- pass 2: gamma along +y, Green functions ----------------
-  {
-    const int baseIn = global(v.idxInG)[col], baseOut = global(v.idxOutG)[col];
-    int cntIn = 0, cntOut = 0;
-    Cx<T> coh[EL];
-#pragma unroll
-    for (int j = 0; j < EL; ++j) coh[j] = {T(0), T(0)};
-    Cx<T> dPrev = {T(0), T(0)};
-    T esPrev = T(0);
-    bool havePrev = false;
-    int8_t lcur = lab[size_t(it.ylo) * N1];
-    // gamma~ of the next site, loaded one site ahead of its use
-    Cx<T> gtNext[EL];
-    const bool green = active && !a.burnin;
-#pragma unroll
-    for (int j = 0; j < EL; ++j) gtNext[j] = {T(0), T(0)};
-    if (green && lcur > 0) {
-#pragma unroll
-      for (int j = 0; j < EL; ++j)
-        gtNext[j] = loadStream(scr + (size_t(len - 1) * EL + j) * 64 + lane);
-    }
-    double nre = 0.0, nim = 0.0, nes = 0.0;
-    int nlab = 0;
-    auto loadChunk = [&](int t0) {
-      const int tt = t0 + g;
-      if (colActive && g < gp && tt < len) {
-        const int y = it.ylo + tt;
-        const size_t fi = size_t(k - v.fieldBase) * n1 + size_t(y) * N1 + x;
-        nre = global(v.fields)[fi];
-        nim = global(v.fields)[v.fieldPlane + fi];
-        nes = global(v.fields)[2 * v.fieldPlane + fi];
-        nlab = lab[size_t(y) * N1];
-      } else {
-        nre = nim = nes = 0.0;
-        nlab = 0;
-      }
-    };
-    loadChunk(0);
-    for (int t0 = 0; t0 < len; t0 += gp) {
-      const double fre = nre, fim = nim, fes = nes;
-      const int flab = nlab;
-      const bool more = t0 + gp < len;
-      if (more) loadChunk(t0 + gp);
-      // at least one site (t0 < len, gp >= 1): with no zero-trip path every
-      // way to the next chunk passes a site's memory operations, and the
-      // wait for this chunk's loads there is counted past them
-      const int tEnd = max(1, min(gp, len - t0));
-      for (int i = 0; i < tEnd; ++i) {
-        const int src = i * cols + c;
-        const double dre = __shfl(fre, src), dim = __shfl(fim, src), e = __shfl(fes, src);
-        const int t = t0 + i;
-        const int y = it.ylo + t;
-        const int ln = i + 1 < tEnd ? __shfl(flab, src + cols) : (more ? __shfl(nlab, c) : 0);
-        const int8_t lnext = int8_t(ln);
-        const Cx<T> D = {T(dre), T(dim)};
-        const T es = T(e);
-        Cx<T> gtCur[EL];
-#pragma unroll
-        for (int j = 0; j < EL; ++j) gtCur[j] = gtNext[j];
-        // Every path through a site issues the same vector memory operations
-        // (this prefetch, then the Green record's two stores): the wait for
-        // the prefetched gamma~ is then counted past the stores that follow
-        // it and leaves them in flight.  A branch around either would make
-        // the count path-dependent, and the wait would also hold for the
-        // store's completion at every site.  Sites that need no gamma~ read
-        // a clamped, valid index of the slot's scratch.
-        {
-          const size_t tn = size_t(max(len - 2 - t, 0));
-#pragma unroll
-          for (int j = 0; j < EL; ++j) gtNext[j] = loadStream(scr + (tn * EL + j) * 64 + lane);
-        }
-        if (active) {
-          if (lcur == 1 || lcur == 3) {
-            const Cx<T> Dm = {(dPrev.re + D.re) * T(0.5), (dPrev.im + D.im) * T(0.5)};
-            const StepSite<T> ps = stepSite(Dm, (esPrev + es) * T(0.5), h);
-            const T half = havePrev ? T(1) : T(0.5);
-#pragma unroll
-            for (int j = 0; j < EL; ++j) coh[j] = stepE<KEL>(ps, ser[j] * half, sej[j] * half, coh[j]);
-            if (lcur == 3) {
-              const int ci = baseOut + cntOut;
-              const T dr = T(global(v.distOutG)[ci]), d = dr * h;
-              const StepSite<T> pe = stepSite(D, es, d);
-#pragma unroll
-              for (int j = 0; j < EL; ++j) {
-                if (!eOk[j]) continue;
-                const Cx<T> bv = stepE<KEL>(pe, ser[j] * dr, sej[j] * dr, coh[j]);
-                const size_t si = size_t(ci) * Ne + g * EL + j;
-                global(v.bOutG)[si] = double(bv.re);
-                global(v.bOutG)[size_t(v.nOutG) * Ne + si] = double(bv.im);
-              }
-              ++cntOut;
-            }
-          } else if (lcur == 2) {
-            const int ci = baseIn + cntIn;
-            const T dr = T(global(v.distInG)[ci]), d = dr * h;
-            const StepSite<T> pe = stepSite(D, es, d);
-#pragma unroll
-            for (int j = 0; j < EL; ++j) {
-              const size_t si = size_t(ci) * Ne + g * EL + j;
-              const GlobalPtr<const double> bin = global(v.bInG);
-              const Cx<T> b0 = eOk[j] ? Cx<T>{T(bin[si]), T(bin[size_t(v.nInG) * Ne + si])}
-                                      : Cx<T>{T(0), T(0)};
-              coh[j] = stepE<KEL>(pe, ser[j] * dr, sej[j] * dr, b0);
-            }
-            ++cntIn;
-          } else {
-#pragma unroll
-            for (int j = 0; j < EL; ++j) coh[j] = {T(0), T(0)};
-          }
-        }
-        // Green functions at inside sites (GreensFunctionStatic.h:125-157,
-        // LocalGreens.h:32-70, ComputeFreeEnergy.h:95-160).  Per energy, with
-        // p = gamma gamma~ and F = 2 i / (1 + p):
-        //   f + f~* = F (gamma~ - gamma) [real part], -F (gamma + gamma~) [imag]
-        //   Re g = Im((1 - p) / (1 + p)) = -2 Im p / |1 + p|^2
-        //   Re i(D* gamma - D gamma~) summed as D.re Su + D.im Sw with
-        //   Su = sum r Im(gamma~ - gamma), Sw = sum r Re(gamma + gamma~).
-        if constexpr (KEL) {
-          // Spectral weight per energy (ComputeLDOS.h:126-151 with
-          // LocalGreens.h:32-45): -Im(i X) with X = -(1 - p) / (1 + p),
-          // i.e. Re((1 - p) / (1 + p)) = (1 - |p|^2) / |1 + p|^2.
-          // Every lane stores its EL weights on every path, as the Green
-          // records below; weights with no site or energy to go to land in
-          // the consumed scratch.
-          const bool record = !a.burnin && lcur > 0 && active;
-          double *const row =
-              v.G + (size_t(k - v.angleBase) * n1 + size_t(y) * N1 + x) * Ne + g * EL;
-          double *const sink = reinterpret_cast<double *>(scr + size_t(len - 1) * EL * 64);
-#pragma unroll
-          for (int j = 0; j < EL; ++j) {
-            double wgt = 0.0;
-            if (record && eOk[j]) {
-              const Cx<T> p = coh[j] * gtCur[j];
-              const T pr = T(1) + p.re;
-              const T den = pr * pr + p.im * p.im;
-              wgt = double((T(1) - (p.re * p.re + p.im * p.im)) * rcpT(den));
-            }
-            *global(record && eOk[j] ? row + j : sink + j) = wgt;
-          }
-        } else {
-          const bool record = !a.burnin && lcur > 0;
-          double gdr = 0.0, gdi = 0.0, gj = 0.0, su = 0.0, sw = 0.0, gf = 0.0;
-          if (record && active) {
-#pragma unroll
-            for (int j = 0; j < EL; ++j) {
-              if (!eOk[j]) continue;
-              const Cx<T> ga = coh[j];
-              const Cx<T> gt = gtCur[j];
-              const Cx<T> p = ga * gt;
-              const T pr = T(1) + p.re;
-              const T r2 = T(2) * rcpT(pr * pr + p.im * p.im);
-              const Cx<T> F = {p.im * r2, pr * r2};
-              const Cx<T> u = gt - ga;
-              const Cx<T> w = ga + gt;
-              const double r = double(res[j]);
-              gdr += r * double(F.re * u.re - F.im * u.im);
-              gdi -= r * double(F.re * w.im + F.im * w.re);
-              gj -= r * double(p.im * r2);
-              su += r * double(u.im);
-              sw += r * double(w.re);
-            }
-          }
-          if (record) {
-            gf = dre * su + dim * sw;
-            // sum the energy groups of this column (lanes c, c + cols, ...)
-            // into lane c: a butterfly when the groups fill the wavefront,
-            // else the other groups' lanes read in turn
-            if (gp * cols == 64) {
-              for (int m = cols; m < 64; m <<= 1) {
-                gdr += __shfl_xor(gdr, m);
-                gdi += __shfl_xor(gdi, m);
-                gj += __shfl_xor(gj, m);
-                gf += __shfl_xor(gf, m);
-              }
-            } else {
-              const double g0r = gdr, g0i = gdi, g0j = gj, g0f = gf;
-              for (int m = 1; m < gp; ++m) {
-                const int src = c + m * cols;
-                gdr += __shfl(g0r, src);
-                gdi += __shfl(g0i, src);
-                gj += __shfl(g0j, src);
-                gf += __shfl(g0f, src);
-              }
-            }
-          }
-          // lanes with no record to write store into the slot scratch of
-          // the first gamma~ this pass consumed (site len - 1, read before
-          // the first store and never again)
-          typedef typename VecOf<double>::type D2;
-          const bool real = record && g == 0 && colActive;
-          D2 *dst = real ? reinterpret_cast<D2 *>(v.G + (size_t(k) * n1 + size_t(y) * N1 + x) * 4)
-                         : reinterpret_cast<D2 *>(scr + size_t(len - 1) * EL * 64);
-          const GlobalPtr<D2> Gk = global(dst);
-          Gk[0] = D2{gdr, gdi};
-          Gk[1] = D2{gj, gf};
-        }
-        dPrev = D;
-        esPrev = es;
-        havePrev = true;
-        lcur = lnext;
-      }
-    }
-  }
-}
-
-// Persistent wavefronts pulling items from the work counter.  The second
-// launch bound asks the compiler for a register budget that leaves room for
-// WAVES wavefronts per SIMD.
-// The views and items come as restrict-qualified parameters as well: the
-// sweep never writes them, and with that known the compiler reads them with
-// scalar loads once per item (in SGPRs, uniform across the wavefront) and
-// reaches the arrays they point at with global (not flat) loads, instead of
-// reloading each field after every store the sweep makes.
-template <typename T, int EL, int WAVES, bool KEL>
-__global__ __launch_bounds__(64, WAVES) void sweepKernel(SweepArgs a,
-                                                          const GrainView *__restrict__ views,
-                                                          const SweepItemDev *__restrict__ items) {
-  Cx<T> *scr = reinterpret_cast<Cx<T> *>(a.scratch) + size_t(blockIdx.x) * a.slotStride;
-  for (;;) {
-    // every lane takes part in the fetch (lane 0 adds one, the others
-    // zero): no branch on the lane index surrounds it, so the compiler
-    // cannot merge it with a lane-0 branch of the item into a loop that
-    // some lanes re-enter without lane 0.  Lane 0's old value is the item,
-    // uniform across the wavefront (the item and its grain view are read
-    // with scalar loads).
-    const int item =
-        __builtin_amdgcn_readfirstlane(atomicAdd(a.counter, threadIdx.x == 0 ? 1 : 0));
-    if (item >= a.numItems) break;
-    const SweepItemDev it = items[item];
-    sweepItem<T, EL, KEL>(a, views[it.grain], it, scr);
-  }
 }
 
 // Homogeneous coherence functions at the exit crossings of one direction

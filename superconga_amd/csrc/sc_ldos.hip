@@ -72,7 +72,11 @@ __global__ void ldosFinishKernel(const int *sites, int numSites, int Ne, long lo
   interval[size_t(e) * n0 + sites[i]] = acc[t];
 }
 
-__global__ void ldosResetCounter(int *c) { *c = 0; }
+__global__ void ldosResetCounter(int *c) {
+  c[0] = 0;
+  c[1] = 0;
+  c[kAgainCount] = 0;
+}
 
 int Grain::ldosChunkAngles() const {
   const Setup &s = *s_;

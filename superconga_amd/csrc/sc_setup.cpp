@@ -1364,22 +1364,36 @@ std::vector<SweepItem> sweepItems(const Setup &s, int cols, int *maxLen) {
   std::vector<SweepItem> items;
   const int N1 = s.N1;
   int mx = 1;
+  // columns with more than one entry of a direction: the crossings are
+  // numbered column by column, so the next column's first one tells
+  std::vector<uint8_t> again(size_t(s.Na) * N1, 0);
+  auto mark = [&](const std::vector<int> &first, long long total) {
+    long long next = total;
+    for (size_t q = again.size(); q-- > 0;) {
+      if (first[q] < 0) continue;
+      if (next - first[q] > 1) again[q] = 1;
+      next = first[q];
+    }
+  };
+  mark(s.idxInG, s.nInG);
+  mark(s.idxInGt, s.nInGt);
   for (int k = 0; k < s.Na; ++k) {
     for (int x0 = s.xmin[k]; x0 <= s.xmax[k]; x0 += cols) {
       const int nc = std::min(cols, s.xmax[k] - x0 + 1);
-      int lo = N1, hi = -1;
+      int lo = N1, hi = -1, more = 0;
       for (int c = 0; c < nc; ++c) {
         const size_t q = size_t(k) * N1 + x0 + c;
         if (s.colFirst[q] < 0) continue;
         lo = std::min(lo, s.colFirst[q]);
         hi = std::max(hi, s.colLast[q]);
+        more |= again[q];
       }
       if (hi < 0) continue;
       // one extra site at each end so that the previous-site values of the
       // first inside site are available (the reference starts at ymin/ymax).
       lo = std::max(lo - 1, s.ymin[k]);
       hi = std::min(hi + 1, s.ymax[k]);
-      items.push_back({k, x0, nc, lo, hi});
+      items.push_back({k, x0, nc, lo, hi, more});
       mx = std::max(mx, hi - lo + 1);
     }
   }

@@ -116,6 +116,7 @@ struct SweepItem {
   int x0;
   int ncols;
   int ylo, yhi;
+  int reentered; // 1: a column with more than one entry of gamma or gamma~
 };
 
 // postprocess_config.json (src/postprocess.cu:118-160,

@@ -6,6 +6,8 @@
 
 namespace scamd {
 
+constexpr int kMaxSweepEL = 16; // most energies per lane of any sweep variant
+
 // Per-grain constants and device pointers consumed by the kernels.
 struct GrainView {
   int N0, N1, Ne, Na, Nc;
@@ -46,7 +48,21 @@ struct GrainView {
 
 struct SweepItemDev {
   int grain, angle, x0, ncols, ylo, yhi;
+  int reentered; // a column with more than one entry of gamma or gamma~
 };
+
+// The sweep's work counters: the next item, the next item to sweep again, how
+// many there are to sweep again, and their numbers.
+constexpr int kAgainCount = 2, kAgainList = 3;
+constexpr int kSweepAgainSlots = 1024; // wavefronts that sweep items again, at most
+
+// Compiled sweep variants: (energies per lane, wavefronts per SIMD), for
+// Matsubara energies and for real-frequency (Keldysh) energies.
+#define SC_SWEEP_VARIANTS(X)                                                         \
+  X(1, 4) X(2, 4) X(3, 3) X(4, 2) X(4, 3) X(4, 4) X(5, 2) X(6, 2) X(7, 1) X(7, 2) X(7, 4)  \
+  X(8, 1) X(8, 2) X(8, 4)                                                            \
+  X(14, 1) X(14, 2) X(16, 1) X(16, 2)
+#define SC_KELDYSH_VARIANTS(X) X(2, 4) X(4, 2) X(4, 3) X(4, 4) X(8, 1) X(8, 2) X(8, 4) X(16, 1)
 
 // One launch sweeps the items of one or several grains (a batch); each item
 // names its grain's view.
@@ -54,8 +70,9 @@ struct SweepArgs {
   const GrainView *views;
   const SweepItemDev *items;
   int numItems;
-  int *counter;
-  void *scratch;       // per slot: [maxLen][EL][64] complex T
+  int *counter; // kAgainList + numItems
+  void *scratch;       // per slot: [maxLen][EL][64] complex T (half of it read and
+                       // written where no column is entered at an odd site)
   long long slotStride; // elements of complex T per slot
   int burnin;
 };
