@@ -378,10 +378,10 @@ void Grain::prepareSweep(int precision) {
   int dev = 0, cus = 0;
   SC_HIP(hipGetDevice(&dev));
   SC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  pl.numSlots = std::max(1, std::min(pl.numItems, pl.slotsPerCU * std::max(cus, 1)));
+  pl.numSlots = sweepSlots(pl.numItems, pl.slotsPerCU * std::max(cus, 1));
   const size_t elemBytes = precision == PREC_FP64 ? sizeof(Cx<double>) : sizeof(Cx<float>);
-  const size_t stride = size_t(pl.maxLen) * pl.el * 64; // complex elements per slot
-  const size_t bytes = size_t(pl.numSlots) * stride * elemBytes;
+  const size_t stride = size_t(pl.maxLen) * pl.el * 64; // complex elements per workgroup
+  const size_t bytes = size_t(pl.numSlots / 2) * stride * elemBytes;
   if (bytes > scratchBytes_) {
     if (dScratch_) (void)hipFree(dScratch_);
     dScratch_ = nullptr;
@@ -887,6 +887,10 @@ void launchSweepVariant(int precision, int el, int waves, const SweepArgs &a, in
   if (!(precision == PREC_FP64 ? launchSweepFp64 : launchSweepMixed)(el, waves, a, slots, stream,
                                                                      keldysh))
     throw std::runtime_error("sweep variant not compiled");
+}
+
+int sweepSlots(int numItems, int most) {
+  return 2 * std::max(1, std::min(numItems, (most + 1) / 2));
 }
 
 void growCounter(int *&counter, size_t &cap, int numItems) {
@@ -1933,7 +1937,7 @@ void Grain::sweepAngles(int precision, bool burnin, int k0, int k1) {
   resetCounter<<<1, 1, 0, stream_>>>(dCounter_);
   SC_HIP(hipEventRecord(ev0_, stream_));
   if (a.numItems > 0)
-    launchSweepVariant(precision, pl.el, pl.waves, a, std::min(pl.numSlots, a.numItems),
+    launchSweepVariant(precision, pl.el, pl.waves, a, sweepSlots(a.numItems, pl.numSlots),
                        stream_, false);
   SC_HIP(hipEventRecord(ev1_, stream_));
 }
@@ -2215,9 +2219,9 @@ void Batch::prepare(int precision, const std::vector<int> &act) {
   int dev = 0, cus = 0;
   SC_HIP(hipGetDevice(&dev));
   SC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  pl.numSlots = std::max(1, std::min(pl.numItems, pl.slotsPerCU * std::max(cus, 1)));
+  pl.numSlots = sweepSlots(pl.numItems, pl.slotsPerCU * std::max(cus, 1));
   const size_t elemBytes = precision == PREC_FP64 ? sizeof(Cx<double>) : sizeof(Cx<float>);
-  const size_t bytes = size_t(pl.numSlots) * size_t(pl.maxLen) * pl.el * 64 * elemBytes;
+  const size_t bytes = size_t(pl.numSlots / 2) * size_t(pl.maxLen) * pl.el * 64 * elemBytes;
   if (bytes > scratchBytes_) {
     if (dScratch_) (void)hipFree(dScratch_);
     dScratch_ = nullptr;

@@ -14,6 +14,9 @@
 
 namespace scamd {
 
+// Wavefronts of a sweep over numItems items, two to an item: an even number, at
+// most `most` rounded up to one.
+int sweepSlots(int numItems, int most);
 // Room for the sweep's work counters over numItems items (no work may be
 // using them).
 void growCounter(int *&counter, size_t &cap, int numItems);

@@ -71,9 +71,9 @@ struct SweepArgs {
   const SweepItemDev *items;
   int numItems;
   int *counter; // kAgainList + numItems
-  void *scratch;       // per slot: [maxLen][EL][64] complex T (half of it read and
-                       // written where no column is entered at an odd site)
-  long long slotStride; // elements of complex T per slot
+  void *scratch;        // per workgroup: [maxLen][EL][64] complex T, half of it used
+                        // where no column is entered at an odd site
+  long long slotStride; // elements of complex T per workgroup
   int burnin;
 };
 
