@@ -114,6 +114,15 @@ template <typename T> __device__ __forceinline__ Cx<T> csqrt(Cx<T> z) {
   return scale(csqrt2(z), T(0.70710678118654752440));
 }
 
+// A value the compiler knows nothing about and, being volatile, forms anew each
+// time it is reached.  Without it the loop invariants of every energy (and the
+// expressions that two steps have in common) are formed once and held: the
+// pass needs some 60 registers more and spills.
+template <typename T> __device__ __forceinline__ void opaque(T &x) { asm volatile("" : "+v"(x)); }
+template <typename T> __device__ __forceinline__ void opaqueScalar(T &x) {
+  asm volatile("" : "+s"(x));
+}
+
 // The sign of every x seen so far: negative once one was.
 __device__ __forceinline__ void noteSign(int &neg, float x) { neg |= __float_as_int(x); }
 __device__ __forceinline__ void noteSign(int &neg, double x) { neg |= __double2hiint(x); }
@@ -140,23 +149,23 @@ template <typename T> __device__ __forceinline__ Cx<T> cdiv(Cx<T> a, Cx<T> b) {
 
 // One implicit-midpoint step of the Riccati equation (RiccatiSolutions.h:65-94):
 // y solves a (y + y0)^2 + (s e - 1) y + (s e + 1) y0 + s D = 0 with s = i h and
-// a = s conj(D) / 4; with disc = (s e - 1)^2 + h^2 |D|^2 - 8 a y0, where only the
-// last term depends on y0, and R = sqrt(disc),
-//   y = y0 + 2 (y0 w + s D) / (2 - w),   w = s e + 1 - R            (FP64)
-//   y = y0 + 4 C / (R - B),   B = s e - 1 + 2 alpha,  alpha = 2 a y0,
-//                             C = (alpha + s e) y0 + s D / 2       (FP32).
-// The two are the same root, solved for the increment of y: the FP32 form
-// rounds nothing that is larger than the increment (over 600 steps of h = 0.05
-// its error against FP64 is 1e-7 of y, that of the root y taken whole 2e-6);
-// the FP64 form takes 1 - R, exact in floating point, for 6 instructions less,
-// and its error is that of the root y taken whole (1e-15 of y) or below.  A step
-// is 42 (FP64) and 32 (FP32) add/multiply instructions, 3 square roots and
-// reciprocals; the root taken whole was 63.
+// a = s conj(D) / 4.  In FP32 it is the quadratic's root taken whole: with
+// b = 2 a y0 + s e - 1, c = (a y0 + s e + 1) y0 + s D,
+//   y = 2 c / (-b + sqrt(b^2 - 4 a c)).
+// In FP64, with disc = b^2 - 4 a c = (s e - 1)^2 + h^2 |D|^2 - 8 a y0, where only
+// the last term depends on y0, and R = sqrt(disc), the same root as an increment:
+//   y = y0 + 2 (y0 w + s D) / (2 - w),   w = s e + 1 - R,
+// 42 add/multiply instructions instead of 63; 1 - R is exact in floating point,
+// and the error is that of the root taken whole (1e-15 of y) or below.
+// FP32 keeps the root: an increment form of 32 instructions is 20 times closer
+// to FP64 (1e-7 of y after 600 steps of h = 0.05, against 2e-6 of the root, whose
+// rounding of 1 - s e acts alike at every step), but the FP32 solution moves by
+// what it gains: by 2e-4 of the current after two runs of an accelerated solve.
 // The quantities that only depend on the site (D, the energy shift Re e and
 // h) are formed once per site and shared by every Ozaki energy.
-// The arithmetic is written with explicit fused multiply-adds, so that every
-// place that takes the same step (a sweep, a segment integrated again from a
-// checkpoint, the adjoint) rounds alike.
+// The FP64 arithmetic is written with explicit fused multiply-adds, so that
+// every place that takes the same step (a sweep, a segment integrated again
+// from a checkpoint, the adjoint) rounds alike.
 template <typename T> struct StepSite;
 
 // FP64: everything but w is scaled so that the quotient needs no factor, disc
@@ -198,44 +207,44 @@ __device__ __forceinline__ Cx<double> stepEnergy(const StepSite<double> &p, doub
           fma(fma(c.im, q.re, c.re * q.im), r, y0.im)};
 }
 
-// FP32: scaled so that the quotient needs no factor, disc by 1/16, R - B by 1/4.
 template <> struct StepSite<float> {
-  Cx<float> a2; // 2 a = i h conj(D) / 2; s D / 2 = (-a2.re, a2.im)
+  Cx<float> a;  // s conj(D) / 4
+  Cx<float> a4; // 4 a
+  Cx<float> sD; // s D = (-4 a.re, 4 a.im)
   float sei;    // Im(s e) = h Re e
-  float sei4;   // sei / 4
-  float k16;    // (h^2 |D|^2 - sei^2) / 16
-  float quarter;
+  float one;
 };
 __device__ __forceinline__ StepSite<float> stepSite(Cx<float> D, float shift, float h) {
-#pragma clang fp contract(off)
   StepSite<float> p;
-  const float hh = 0.5f * h;
-  p.a2 = {hh * D.im, hh * D.re};
+  p.a4 = {h * D.im, h * D.re};
+  p.a = {0.25f * p.a4.re, 0.25f * p.a4.im};
+  p.sD = {-p.a4.re, p.a4.im};
   p.sei = h * shift;
-  p.sei4 = 0.25f * p.sei;
-  p.k16 = fmaf(0.25f, fmaf(p.a2.re, p.a2.re, p.a2.im * p.a2.im), -(p.sei4 * p.sei4));
-  p.quarter = 0.25f;
+  p.one = 1.f;
   return p;
+}
+// The principal root with Kahan's selects: of any discriminant, WHOLE or not.
+__device__ __forceinline__ Cx<float> rootOfStep(Cx<float> z) {
+  const float n = fmax(z.re * z.re + z.im * z.im, std::numeric_limits<float>::min());
+  const float m = n * rsqT(n);
+  const float u = 0.5f * (fabs(z.re) + m);
+  const float r = rsqT(u);
+  const float t = u * r;
+  const float q = (0.5f * z.im) * r;
+  const bool right = z.re >= 0.f;
+  return {right ? t : fabs(q), right ? q : copysign(t, z.im)};
 }
 template <bool WHOLE>
 __device__ __forceinline__ Cx<float> stepEnergy(const StepSite<float> &p, float ser, Cx<float> y0,
-                                                int &neg) {
-#pragma clang fp contract(off)
-  const Cx<float> al = {fmaf(p.a2.re, y0.re, -(p.a2.im * y0.im)),
-                        fmaf(p.a2.re, y0.im, p.a2.im * y0.re)};
-  const Cx<float> v = {al.re + ser, al.im + p.sei};
-  const Cx<float> c = {fmaf(v.re, y0.re, fmaf(-v.im, y0.im, -p.a2.re)),
-                       fmaf(v.re, y0.im, fmaf(v.im, y0.re, p.a2.im))};
-  const float b = fmaf(p.quarter, ser, -p.quarter); // (Re(s e) - 1) / 4
-  const Cx<float> z = {fmaf(-p.quarter, al.re, fmaf(b, b, p.k16)),
-                       fmaf(-p.quarter, al.im, (2.f * p.sei4) * b)};
-  const Cx<float> R = stepRoot2<WHOLE>(z, neg); // sqrt(2 disc) / 4
-  constexpr float kHalfRoot = 0.70710678118654752440f;
-  const Cx<float> q = {fmaf(kHalfRoot, R.re, -fmaf(0.5f, al.re, b)),
-                       fmaf(kHalfRoot, R.im, -fmaf(0.5f, al.im, p.sei4))};
-  const float r = rcpT(fmaf(q.re, q.re, q.im * q.im));
-  return {fmaf(fmaf(c.re, q.re, c.im * q.im), r, y0.re),
-          fmaf(fmaf(c.im, q.re, -(c.re * q.im)), r, y0.im)};
+                                                int &) {
+  const Cx<float> ay = p.a * y0;
+  const Cx<float> b = {2.f * ay.re + (ser - p.one), 2.f * ay.im + p.sei};
+  const Cx<float> t = {ay.re + (ser + p.one), ay.im + p.sei};
+  const Cx<float> c = t * y0 + p.sD;
+  const Cx<float> ac4 = p.a4 * c;
+  const Cx<float> disc = {b.re * b.re - b.im * b.im - ac4.re, 2.f * b.re * b.im - ac4.im};
+  const Cx<float> sq = rootOfStep(disc);
+  return cdiv(c + c, sq - b);
 }
 
 // Real-frequency energies eps = E + i delta: sej = h E joins the site's
@@ -254,8 +263,6 @@ __device__ __forceinline__ Cx<float> stepEnergy(const StepSite<float> &p, float 
                                                 Cx<float> y0, int &neg) {
   StepSite<float> e = p;
   e.sei = p.sei + sej;
-  e.sei4 = 0.25f * e.sei;
-  e.k16 = fmaf(p.sei4 - e.sei4, p.sei4 + e.sei4, p.k16);
   return stepEnergy<WHOLE>(e, ser, y0, neg);
 }
 // a step from any y0

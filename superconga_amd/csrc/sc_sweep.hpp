@@ -68,14 +68,6 @@ __device__ __forceinline__ double pairSum16(double a, double b) {
   return __builtin_bit_cast(double, x) + __builtin_bit_cast(double, y);
 }
 
-// A value the compiler knows nothing about and, being volatile, forms anew each
-// time it is reached.  Without it the loop invariants of every energy (and the
-// expressions that two steps have in common) are formed once and held: the
-// pass needs some 60 registers more and spills.
-template <typename T> __device__ __forceinline__ void opaque(T &x) { asm volatile("" : "+v"(x)); }
-template <typename T> __device__ __forceinline__ void opaqueScalar(T &x) {
-  asm volatile("" : "+s"(x));
-}
 __device__ __forceinline__ StepSite<double> apart(StepSite<double> p) {
   opaque(p.a4.re);
   opaque(p.a4.im);
@@ -85,11 +77,12 @@ __device__ __forceinline__ StepSite<double> apart(StepSite<double> p) {
   return p;
 }
 __device__ __forceinline__ StepSite<float> apart(StepSite<float> p) {
-  opaque(p.a2.re);
-  opaque(p.a2.im);
-  opaque(p.sei4);
-  opaque(p.k16);
-  opaqueScalar(p.quarter);
+  opaque(p.a4.re);
+  opaque(p.a4.im);
+  opaque(p.sei);
+  p.a = {0.25f * p.a4.re, 0.25f * p.a4.im};
+  p.sD = {-p.a4.re, p.a4.im};
+  opaqueScalar(p.one);
   return p;
 }
 // only what the energies form of the constant apart; the constant of q
@@ -98,7 +91,7 @@ __device__ __forceinline__ StepSite<double> fresh(StepSite<double> p) {
   return p;
 }
 __device__ __forceinline__ StepSite<float> fresh(StepSite<float> p) {
-  opaqueScalar(p.quarter);
+  opaqueScalar(p.one);
   return p;
 }
 __device__ __forceinline__ StepSite<double> alike(StepSite<double> p, const StepSite<double> &q) {
@@ -106,7 +99,7 @@ __device__ __forceinline__ StepSite<double> alike(StepSite<double> p, const Step
   return p;
 }
 __device__ __forceinline__ StepSite<float> alike(StepSite<float> p, const StepSite<float> &q) {
-  p.quarter = q.quarter;
+  p.one = q.one;
   return p;
 }
 // the step of gamma~ (-conj(D)) where p is that of gamma, and the other way
@@ -115,7 +108,9 @@ __device__ __forceinline__ StepSite<double> tilde(StepSite<double> p) {
   return p;
 }
 __device__ __forceinline__ StepSite<float> tilde(StepSite<float> p) {
-  p.a2.im = -p.a2.im;
+  p.a.im = -p.a.im;
+  p.a4.im = -p.a4.im;
+  p.sD.im = -p.sD.im;
   return p;
 }
 
