@@ -423,6 +423,11 @@ __device__ __forceinline__ bool sweepItem(const SweepArgs &a, const GrainView &v
         o[1] = D2{s[2], s[3]};
       }
     };
+    // An even energy's weight waits for the next one's where both fit one
+    // 16-byte store (EL and Ne even): half the stores, each to a line of its
+    // own per lane.
+    double held = 0.0;
+    const bool twos = EL % 2 == 0 && Ne % 2 == 0;
     auto putWeight = [&](int j, Cx<T> ga, Cx<T> gt, const SiteRow &f, int y) {
       const Cx<T> p = ga * gt;
       const T pr = T(1) + p.re;
@@ -430,7 +435,14 @@ __device__ __forceinline__ bool sweepItem(const SweepArgs &a, const GrainView &v
       const bool record = !a.burnin && f.lab > 0 && real && e0 + j < Ne;
       double *const dst = record ? Gk + (size_t(y) * N1 + x) * Ne + e0 + j
                                  : reinterpret_cast<double *>(sink);
-      *global(dst) = double(wgt);
+      if (!twos) {
+        *global(dst) = double(wgt);
+      } else if (j % 2 == 0) {
+        held = double(wgt);
+      } else {
+        typedef typename VecOf<double>::type D2;
+        *global(reinterpret_cast<D2 *>(record ? dst - 1 : dst)) = D2{held, double(wgt)};
+      }
     };
 
     // the other one's even site t of a pair; each energy's next one is loaded
