@@ -283,6 +283,78 @@ bool sweepVariantExists(int el, int waves, bool keldysh) {
   return false;
 }
 
+// The lane layout of a sweep whose caller sets none.  Fewer energies per lane
+// give more wavefronts, which a small grain needs to fill the chip and which
+// shorten the step of the chain that bounds it; more of them share a site's
+// fields and sums, and a count that divides the grain's leaves no lane
+// padding.  Per layout the time is estimated as that of the longest chain,
+// maxLen (latency + latencyPer el), or of all wavefronts' instructions over
+// the 1024 SIMDs, rows / 512 issue (el + shared), whichever is larger (FP32,
+// whose instructions leave a SIMD more room: their cubes added).  The
+// coefficients are fitted to measured times of 14 grains (discs, squares and
+// octagons of 46 to 930 sites a side, 7 to 28 energies, 16 to 128 angles):
+// the layout picked is within 2% (FP64) and 8% (FP32) of the fastest of all
+// compiled ones there, where one layout for all, 8 energies a lane at two
+// wavefronts per SIMD, is up to 2.6 times slower (0.120 against 0.047 ms on
+// the smallest) and 13% and 19% on the largest (20.9 against 18.4 ms in FP64,
+// 15.2 against 12.7 in FP32).
+SweepShape defaultSweepShape(const std::vector<const Setup *> &grains, int precision) {
+  const bool dp = precision == PREC_FP64;
+  const double latency = 3.0, latencyPer = dp ? 1.2 : 0.2, issue = dp ? 1.6 : 0.2;
+  const double shared = dp ? 0.6 : 1.5, sharedLess = dp ? 0.2 : 1.0;
+  // compiled without register spills (or nearly: 3 at three wavefronts)
+  const SweepShape fp64[] = {{1, 4, 16}, {3, 3, 16}, {4, 2, 16}, {5, 2, 16}, {6, 2, 16}, {7, 2, 8},
+                             {8, 2, 8}};
+  const SweepShape fp32[] = {{1, 4, 16}, {2, 4, 16}, {3, 3, 16}, {4, 2, 16}, {5, 2, 16},
+                             {6, 2, 16}, {7, 2, 16}, {8, 2, 16}};
+  SweepShape best{8, 2, 8};
+  double least = -1.0;
+  const SweepShape *all = dp ? fp64 : fp32;
+  const int count = dp ? int(sizeof(fp64) / sizeof(fp64[0])) : int(sizeof(fp32) / sizeof(fp32[0]));
+  for (int i = 0; i < count; ++i) {
+    const int el = all[i].el;
+    double chain = 0.0, work = 0.0;
+    bool fits = true;
+    for (const Setup *s : grains) {
+      const int groups = (s->Ne + el - 1) / el;
+      if (groups > 64) {
+        fits = false;
+        break;
+      }
+      const int cols = 64 / groups;
+      long long rows = 0;
+      int maxLen = 0;
+      sweepLoad(*s, cols, rows, maxLen);
+      // one lane per column, or four: the sums of a site need fewest exchanges
+      const bool less = groups == 1 || (groups == 4 && cols == 16);
+      chain = std::max(chain, maxLen * (latency + latencyPer * el));
+      work += double(rows) / 512.0 * issue * (el + (less ? sharedLess : shared));
+    }
+    if (!fits) continue;
+    const double t = dp ? std::max(chain, work) : std::cbrt(chain * chain * chain + work * work * work);
+    if (least < 0.0 || t < least) {
+      least = t;
+      best = all[i];
+    }
+  }
+  return best;
+}
+
+void Grain::chooseSweepShape(int precision) {
+  SweepPlan &pl = plan_[precision];
+  if (pl.shapeSet) return;
+  SweepShape sh{8, 2, 8};
+  if (!s_->keldysh)
+    sh = defaultSweepShape({s_.get()}, precision);
+  else if (s_->Ne <= 4 * 64)
+    // real energies: 4 a lane on every grain measured (discs of 56 to 606
+    // sites a side, 16 to 33 energies, 90 to 720 angles), 4 to 41% faster
+    // than 8 a lane (FP64 14.3 against 15.4 ms and 0.173 against 0.295, FP32
+    // 9.2 against 10.8 and 0.143 against 0.209)
+    sh = precision == PREC_FP64 ? SweepShape{4, 2, 16} : SweepShape{4, 3, 16};
+  setSweepShape(precision, sh.el, sh.waves, sh.slotsPerCU);
+}
+
 void Grain::setSweepShape(int precision, int el, int waves, int slotsPerCU) {
   if (precision != PREC_FP64 && precision != PREC_MIXED)
     throw std::runtime_error("unknown precision");
@@ -297,9 +369,11 @@ void Grain::setSweepShape(int precision, int el, int waves, int slotsPerCU) {
   pl.el = el;
   pl.waves = waves;
   pl.slotsPerCU = slotsPerCU;
+  pl.shapeSet = true;
 }
 
-void Grain::sweepShape(int precision, int &el, int &waves, int &slotsPerCU) const {
+void Grain::sweepShape(int precision, int &el, int &waves, int &slotsPerCU) {
+  chooseSweepShape(precision == PREC_FP64 ? 0 : 1);
   const SweepPlan &pl = plan_[precision == PREC_FP64 ? 0 : 1];
   el = pl.el;
   waves = pl.waves;
@@ -307,6 +381,7 @@ void Grain::sweepShape(int precision, int &el, int &waves, int &slotsPerCU) cons
 }
 
 void Grain::prepareSweep(int precision) {
+  chooseSweepShape(precision);
   SweepPlan &pl = plan_[precision];
   if (pl.ready) return;
   // the buffers below may still be read by a sweep in flight
@@ -934,10 +1009,10 @@ void Grain::autotune(int precision) {
   }
   ensureBoundaryInit();
   extendDelta();
-  SweepPlan &pl = plan_[precision];
-  const int keepEl = pl.el, keepW = pl.waves, keepSlots = pl.slotsPerCU;
+  chooseSweepShape(precision);
+  const SweepPlan &pl = plan_[precision];
   float best = -1.f;
-  int bestEl = keepEl, bestW = keepW, bestSlots = keepSlots;
+  int bestEl = pl.el, bestW = pl.waves, bestSlots = pl.slotsPerCU;
   const int slotChoices[] = {4, 8, 16};
   auto tryShape = [&](int el, int w, int slots) {
     if ((s_->Ne + el - 1) / el > 64) return;
@@ -967,9 +1042,6 @@ void Grain::autotune(int precision) {
   }
 #undef SC_TRY
   setSweepShape(precision, bestEl, bestW, bestSlots);
-  (void)keepEl;
-  (void)keepW;
-  (void)keepSlots;
 }
 
 void Grain::queueBoundaryCondition(int handles[2]) {
@@ -2144,9 +2216,20 @@ void Batch::setSweepShape(int precision, int el, int waves, int slotsPerCU) {
   pl.el = el;
   pl.waves = waves;
   pl.slotsPerCU = slotsPerCU;
+  pl.shapeSet = true;
 }
 
-void Batch::sweepShape(int precision, int &el, int &waves, int &slotsPerCU) const {
+void Batch::chooseSweepShape(int precision) {
+  if (plan_[precision].shapeSet) return;
+  // for all grains, whichever are still iterating
+  std::vector<const Setup *> all;
+  for (auto &g : grains_) all.push_back(&g->setup());
+  const SweepShape sh = defaultSweepShape(all, precision);
+  setSweepShape(precision, sh.el, sh.waves, sh.slotsPerCU);
+}
+
+void Batch::sweepShape(int precision, int &el, int &waves, int &slotsPerCU) {
+  chooseSweepShape(precision == PREC_FP64 ? 0 : 1);
   const Plan &pl = plan_[precision == PREC_FP64 ? 0 : 1];
   el = pl.el;
   waves = pl.waves;
@@ -2154,6 +2237,7 @@ void Batch::sweepShape(int precision, int &el, int &waves, int &slotsPerCU) cons
 }
 
 void Batch::prepare(int precision, const std::vector<int> &act) {
+  chooseSweepShape(precision);
   Plan &pl = plan_[precision];
   if (pl.ready && pl.key == act) return;
   SC_HIP(hipStreamSynchronize(stream_));

@@ -14,6 +14,12 @@
 
 namespace scamd {
 
+// A lane layout of the sweep: energies per lane, wavefronts per SIMD the
+// variant is compiled for, persistent wavefronts per compute unit.
+struct SweepShape {
+  int el, waves, slotsPerCU;
+};
+SweepShape defaultSweepShape(const std::vector<const Setup *> &grains, int precision);
 // Wavefronts of a sweep over numItems items, two to an item: an even number, at
 // most `most` rounded up to one.
 int sweepSlots(int numItems, int most);
@@ -172,8 +178,9 @@ public:
   // register budget (wavefronts per SIMD the kernel is compiled for) and
   // persistent wavefronts per compute unit.
   void setSweepShape(int precision, int energiesPerLane, int wavesPerSimd, int slotsPerCU);
-  void sweepShape(int precision, int &energiesPerLane, int &wavesPerSimd,
-                  int &slotsPerCU) const;
+  void sweepShape(int precision, int &energiesPerLane, int &wavesPerSimd, int &slotsPerCU);
+  // the lane layout by size, where the caller has set none
+  void chooseSweepShape(int precision);
   // Times every compiled sweep variant on the current state and keeps the
   // fastest for `precision`; the sweeps it runs leave the state unchanged.
   void autotune(int precision);
@@ -447,6 +454,7 @@ private:
   // sweep plans, one per precision
   struct SweepPlan {
     int el = 8, waves = 2, slotsPerCU = 8;
+    bool shapeSet = false; // by the caller or chooseSweepShape
     int cols = 0, groups = 0, maxLen = 0, numItems = 0, numSlots = 0;
     // Keldysh: items grouped by angle chunk (chunkAngles frames each),
     // chunk c's items at [chunkStart[c], chunkStart[c + 1])
@@ -573,7 +581,9 @@ public:
   // number converged.
   int run(int nBurnin, int itMin, int itMax, int precision, std::vector<int> &converged);
   void setSweepShape(int precision, int el, int waves, int slotsPerCU);
-  void sweepShape(int precision, int &el, int &waves, int &slotsPerCU) const;
+  void sweepShape(int precision, int &el, int &waves, int &slotsPerCU);
+  // the lane layout by size, where the caller has set none
+  void chooseSweepShape(int precision);
   void autotune(int precision);
   double lastSweepMs() const { return sweepMs_; }
   double lastIterationMs() const { return iterMs_; }
@@ -590,6 +600,7 @@ public:
 private:
   struct Plan {
     int el = 8, waves = 2, slotsPerCU = 8;
+    bool shapeSet = false; // by the caller or chooseSweepShape
     std::vector<int> key; // the active grains the items were built for
     int numItems = 0, numSlots = 0, maxLen = 0;
     void *dItems = nullptr, *dViews = nullptr;

@@ -1426,6 +1426,26 @@ std::unique_ptr<Setup> buildSetup(const Config &cfg) {
   return sp;
 }
 
+void sweepLoad(const Setup &s, int cols, long long &rows, int &maxLen) {
+  // the rows of the items sweepItems makes
+  rows = 0;
+  maxLen = 1;
+  for (int k = 0; k < s.Na; ++k)
+    for (int x0 = s.xmin[k]; x0 <= s.xmax[k]; x0 += cols) {
+      int lo = s.N1, hi = -1;
+      for (int x = x0; x < std::min(x0 + cols, s.xmax[k] + 1); ++x) {
+        const size_t q = size_t(k) * s.N1 + x;
+        if (s.colFirst[q] < 0) continue;
+        lo = std::min(lo, s.colFirst[q]);
+        hi = std::max(hi, s.colLast[q]);
+      }
+      if (hi < 0) continue;
+      const int len = std::min(hi + 1, s.ymax[k]) - std::max(lo - 1, s.ymin[k]) + 1;
+      rows += len;
+      maxLen = std::max(maxLen, len);
+    }
+}
+
 std::vector<SweepItem> sweepItems(const Setup &s, int cols, int *maxLen) {
   std::vector<SweepItem> items;
   const int N1 = s.N1;

@@ -190,6 +190,9 @@ void setKeldyshBlock(Setup &s, int start);
 std::vector<SweepItem> sweepItems(const Setup &s, int colsPerItem,
                                   int *maxLength);
 
+// Rows over all items of that work list, and the longest item's.
+void sweepLoad(const Setup &s, int colsPerItem, long long &rows, int &maxLength);
+
 // Stand-alone pieces exposed through the C ABI for unit checks.
 int numOzakiEnergies(double temperature, double cutoff);
 void ozakiPoles(int numPoles, std::vector<double> &poles,
