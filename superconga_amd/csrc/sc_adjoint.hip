@@ -46,7 +46,7 @@ namespace scamd {
 namespace {
 
 constexpr int kAdjEL = kAdjointEL; // Ozaki energies per lane of the reverse sweep
-constexpr int kAdjSlotsPerCU = 8; // persistent wavefronts per compute unit (2 per SIMD)
+constexpr int kAdjWaves = 2; // persistent wavefronts per SIMD
 
 __device__ __forceinline__ Cx<double> conjc(Cx<double> a) { return {a.re, -a.im}; }
 
@@ -87,6 +87,40 @@ __device__ __forceinline__ Cx<double> stepAdjoint(const StepSite<double> &p, dou
   const Cx<double> qiw = q * Cx<double>{-w.im, w.re};
   ebar += hs * (qiw.re * ybar.re + qiw.im * ybar.im);
   return conjc(q * fy0) * ybar;
+}
+
+// The adjoint of a step as stepAdjoint takes it, with what the energies of a
+// lane have in common summed before it is multiplied: with the adjoint s of s D
+// and the adjoint conj(w^2) s of a, w = y + y0.
+struct AdjointSums {
+  Cx<double> s = {0.0, 0.0}, a = {0.0, 0.0};
+  double e = 0.0;
+  // dF/dD and dF/des of the step, of length hs
+  __device__ __forceinline__ SiteBar bar(double hs) const {
+    return {hs * (0.25 * a.im + s.im), hs * (0.25 * a.re - s.re), hs * e};
+  }
+};
+__device__ __forceinline__ Cx<double> stepAdjointSums(const StepSite<double> &p, double ser,
+                                                      Cx<double> y0, Cx<double> y,
+                                                      Cx<double> ybar, AdjointSums &t) {
+  const Cx<double> w = y + y0;
+  const Cx<double> a2 = {0.5 * p.a4.re, 0.5 * p.a4.im}; // 2 a
+  double one = 1.0;
+  opaqueScalar(one); // ser - 1 is not worth a register of every energy
+  const Cx<double> fy = {fma(a2.re, w.re, fma(-a2.im, w.im, ser - one)),
+                         fma(a2.re, w.im, fma(a2.im, w.re, p.sei))};
+  const double fy0 = fy.re + 2.0; // with the imaginary part of fy
+  const double r = rcpT(fma(fy.re, fy.re, fy.im * fy.im));
+  const Cx<double> u = {ybar.re * r, ybar.im * r};
+  // s = conj(-1 / F_y) ybar
+  const Cx<double> s = {fma(fy.im, u.im, -(fy.re * u.re)), -fma(fy.re, u.im, fy.im * u.re)};
+  const Cx<double> w2 = {fma(w.re, w.re, -(w.im * w.im)), 2.0 * (w.re * w.im)};
+  t.s.re += s.re;
+  t.s.im += s.im;
+  t.a.re = fma(w2.re, s.re, fma(w2.im, s.im, t.a.re));
+  t.a.im = fma(w2.re, s.im, fma(-w2.im, s.re, t.a.im));
+  t.e = fma(w.re, s.im, fma(-w.im, s.re, t.e));
+  return {fma(fy0, s.re, fy.im * s.im), fma(fy0, s.im, -(fy.im * s.re))};
 }
 
 // Sum over the energy groups of a column (lanes c, c + cols, ...) into the
@@ -301,6 +335,7 @@ struct AdjointArgs {
   double *partial;        // per item: its share of the free-energy sum
   int ck;                 // checkpoint segment length (0: every site kept)
   int ckSeg;              // segments per scratch buffer (ceil(maxLen / ck))
+  int maxLen;             // of the items
 };
 
 // Local adjoints of gamma and gamma~ at one site and energy through the
@@ -325,13 +360,12 @@ __device__ __forceinline__ void greensAdjoint(Cx<double> g, Cx<double> gt, Cx<do
   gtbar = Cx<double>{r, 0.0} * (conjc(Qg * g) * db + conjc(Q * db) + conjc(Qg) * jbc);
 }
 
-// 2. The reverse sweep of one item (the sweep's items and lane layout).
-// RES: the residual mode, seeded from a.seed through greensAdjoint instead
-// of the free-energy density; pass 2 leaves the local adjoint of gamma in
-// the gamma~ scratch (read there already) for pass 3.
-template <int EL, bool RES>
-__device__ void adjointItem(const AdjointArgs &a, const SweepItemDev &it, int itemIndex,
-                            Cx<double> *scrT, Cx<double> *scrG) {
+// 2 (residual). The reverse sweep of one item (the sweep's items and lane
+// layout), seeded from a.seed through greensAdjoint; pass 2 leaves the local
+// adjoint of gamma in the gamma~ scratch (read there already) for pass 3.
+template <int EL>
+__device__ void adjointItem(const AdjointArgs &a, const SweepItemDev &it, Cx<double> *scrT,
+                            Cx<double> *scrG) {
   const GrainView &v = a.view;
   const int lane = threadIdx.x;
   const int cols = v.cols, gp = v.groups;
@@ -346,8 +380,7 @@ __device__ void adjointItem(const AdjointArgs &a, const SweepItemDev &it, int it
   const bool active = colActive && g < gp;
   const int8_t *lab = v.labels + size_t(k) * n1 + x;
   const double *F = v.fields + size_t(k - v.fieldBase) * n1 + x;
-  const double *rhoK = a.rho + size_t(k) * n1 + x;
-  const double *seedK = RES ? a.seed + size_t(k) * n1 + x : nullptr;
+  const double *seedK = a.seed + size_t(k) * n1 + x;
   double *dbK = a.dbar + size_t(k) * n1 + x;
   double ser[EL], res[EL];
   bool eOk[EL];
@@ -531,7 +564,6 @@ __device__ void adjointItem(const AdjointArgs &a, const SweepItemDev &it, int it
   // ------- pass 2: gamma from the bottom, kept; the adjoint of gamma~ -------
   // (B = the site below, processed in the previous iteration)
   int numEntryG = 0;
-  double omega = 0.0;
   {
     const int baseInG = v.idxInG[col], baseInT = v.idxInGt[col];
     int seenT = 0;
@@ -550,7 +582,6 @@ __device__ void adjointItem(const AdjointArgs &a, const SweepItemDev &it, int it
       const double dre = F[o], dim = F[v.fieldPlane + o], es = F[2 * v.fieldPlane + o];
       const Cx<double> D = {dre, dim}, Dt = {-dre, dim};
       const int8_t lc = lab[o];
-      const double rho = RES ? 0.0 : rhoK[o];
       if (K > 0 && (t == len - 1 || t % K == K - 1)) {
         // the bottom of a segment: gamma's state before it, for pass 3, and
         // gamma~ of the segment again
@@ -594,20 +625,8 @@ __device__ void adjointItem(const AdjointArgs &a, const SweepItemDev &it, int it
 #pragma unroll
           for (int j = 0; j < EL; ++j) scrG[slot(t, j)] = coh[j];
         }
-        if constexpr (!RES) {
-          // the free-energy density and its own dependence on D
-          double su = 0.0, sw = 0.0;
-#pragma unroll
-          for (int j = 0; j < EL; ++j) {
-            if (!eOk[j]) continue;
-            su += res[j] * (gt[j].im - coh[j].im);
-            sw += res[j] * (coh[j].re + gt[j].re);
-          }
-          omega += rho * (dre * su + dim * sw);
-          dbCur = {rho * su, rho * sw, 0.0};
-        }
         // adjoint of gamma~ here: what the step into the site below carries
-        // back, plus dF/dgt = rho r (D.im + i D.re)
+        // back, plus the local adjoint
         Cx<double> carry[EL];
 #pragma unroll
         for (int j = 0; j < EL; ++j) carry[j] = {0.0, 0.0};
@@ -624,21 +643,14 @@ __device__ void adjointItem(const AdjointArgs &a, const SweepItemDev &it, int it
           addBar(dbCur, dd, 0.5 * eb);
           addBar(dbB, dd, 0.5 * eb);
         }
-        if constexpr (RES) {
-          const Cx<double> sd = {seedK[o], seedK[a.framePlane + o]};
-          const double sj = seedK[2 * a.framePlane + o];
+        const Cx<double> sd = {seedK[o], seedK[a.framePlane + o]};
+        const double sj = seedK[2 * a.framePlane + o];
 #pragma unroll
-          for (int j = 0; j < EL; ++j) {
-            Cx<double> lg = {0.0, 0.0}, lt = {0.0, 0.0};
-            if (eOk[j]) greensAdjoint(coh[j], gt[j], sd, sj, res[j], lg, lt);
-            mu[j] = eOk[j] ? carry[j] + lt : Cx<double>{0.0, 0.0};
-            if (K == 0) scrT[slot(t, j)] = lg;
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < EL; ++j)
-            mu[j] = eOk[j] ? carry[j] + Cx<double>{rho * res[j] * dim, rho * res[j] * dre}
-                           : Cx<double>{0.0, 0.0};
+        for (int j = 0; j < EL; ++j) {
+          Cx<double> lg = {0.0, 0.0}, lt = {0.0, 0.0};
+          if (eOk[j]) greensAdjoint(coh[j], gt[j], sd, sj, res[j], lg, lt);
+          mu[j] = eOk[j] ? carry[j] + lt : Cx<double>{0.0, 0.0};
+          if (K == 0) scrT[slot(t, j)] = lg;
         }
         // gamma~ entered here from its in-value (the entries in reverse order)
         if (lc == 3) {
@@ -701,12 +713,11 @@ __device__ void adjointItem(const AdjointArgs &a, const SweepItemDev &it, int it
       const double dre = F[o], dim = F[v.fieldPlane + o], es = F[2 * v.fieldPlane + o];
       const Cx<double> D = {dre, dim};
       const int8_t lc = lab[o];
-      const double rho = RES ? 0.0 : rhoK[o];
       if (K > 0 && t % K == 0) {
         // the top of a segment: gamma of the segment again (and, for the
         // residual's local adjoints, gamma~)
         recomputeG(t / K);
-        if constexpr (RES) recomputeT(t / K);
+        recomputeT(t / K);
       }
       Cx<double> gc[EL];
 #pragma unroll
@@ -731,28 +742,20 @@ __device__ void adjointItem(const AdjointArgs &a, const SweepItemDev &it, int it
           addBar(dbCur, dd, 0.5 * eb);
           addBar(dbA, dd, 0.5 * eb);
         }
-        if constexpr (RES) {
-          // the local adjoint of gamma: left by pass 2 in the gamma~ scratch,
-          // or formed here from the segment's gamma~ again
-          const Cx<double> sd = {seedK[o], seedK[a.framePlane + o]};
-          const double sj = seedK[2 * a.framePlane + o];
+        // the local adjoint of gamma: left by pass 2 in the gamma~ scratch,
+        // or formed here from the segment's gamma~ again
+        const Cx<double> sd = {seedK[o], seedK[a.framePlane + o]};
+        const double sj = seedK[2 * a.framePlane + o];
 #pragma unroll
-          for (int j = 0; j < EL; ++j) {
-            Cx<double> lg = {0.0, 0.0};
-            if (K == 0) {
-              lg = scrT[slot(t, j)];
-            } else if (eOk[j]) {
-              Cx<double> lt;
-              greensAdjoint(gc[j], scrT[segSlot(t - (t / K) * K, j)], sd, sj, res[j], lg, lt);
-            }
-            lam[j] = eOk[j] ? carry[j] + lg : Cx<double>{0.0, 0.0};
+        for (int j = 0; j < EL; ++j) {
+          Cx<double> lg = {0.0, 0.0};
+          if (K == 0) {
+            lg = scrT[slot(t, j)];
+          } else if (eOk[j]) {
+            Cx<double> lt;
+            greensAdjoint(gc[j], scrT[segSlot(t - (t / K) * K, j)], sd, sj, res[j], lg, lt);
           }
-        } else {
-          // dF/dg = rho r (D.im - i D.re)
-#pragma unroll
-          for (int j = 0; j < EL; ++j)
-            lam[j] = eOk[j] ? carry[j] + Cx<double>{rho * res[j] * dim, -rho * res[j] * dre}
-                            : Cx<double>{0.0, 0.0};
+          lam[j] = eOk[j] ? carry[j] + lg : Cx<double>{0.0, 0.0};
         }
         // gamma entered here from its in-value (the entries in reverse order)
         if (lc == 2) {
@@ -793,17 +796,286 @@ __device__ void adjointItem(const AdjointArgs &a, const SweepItemDev &it, int it
     }
     writeDbar(it.ylo, dbA, true);
   }
-
-  // this item's share of the free-energy sum.  The butterfly leaves the
-  // same bits in every lane (each level adds the same two operands, only
-  // swapped), so every lane stores it: a store behind a lane-0 branch here
-  // and the lane-0 fetch of the next item were threaded by the compiler
-  // into one path that let lanes 1-63 re-enter the item loop without lane 0.
-  for (int m = 1; m < 64; m <<= 1) omega += __shfl_xor(omega, m);
-  a.partial[itemIndex] = omega;
 }
 
-template <int EL, bool RES>
+// 2 (free energy). The reverse sweep of one recurrence along one item, gamma~
+// from the top (`up` false) or gamma from the bottom: the free-energy density is
+// linear in gamma and gamma~, so the two have nothing in common but dF/dD, to
+// which each adds its part (two additions to zero at a site: the same sum in
+// either order).  Sites are counted from the recurrence's own end.
+//
+// The forward pass keeps the state before every kGradSeg-th site, with the
+// labels of the segment and the crossings before it; the reverse pass takes a
+// segment again, its states and site fields in registers, and runs back over it.
+//
+// What bounds it: a step is 49 FP64 instructions, its adjoint 40, and keeping
+// and reading a state 32 bytes.  One wavefront that went down, up and down again,
+// with checkpoints every sqrt(length) sites and the segments in the scratch, took
+// some 300 instructions and 64 bytes per site and energy of both recurrences in
+// one chain of three passes; this takes 2 (49 + 49 + 40) and 2 * 32 / kGradSeg
+// in two independent chains of two.  A square of 606 sites a side, 12 energies,
+// 128 angles: 19.0 ms before, 11.4 with it.  Segments of 6 sites need 57 registers
+// more than the 256 of two wavefronts a SIMD.
+constexpr int kGradSeg = 4;   // sites of a segment
+constexpr int kGradWaves = 2; // wavefronts per SIMD
+// complex elements of a slot's scratch
+__host__ __device__ inline long long gradientStride(int maxLen) {
+  const long long segs = (maxLen + kGradSeg - 1) / kGradSeg;
+  return segs * (kAdjEL * 64) + (segs * 64 * int(sizeof(int)) + 15) / 16;
+}
+
+template <int EL>
+__device__ __forceinline__ void gradientItem(const AdjointArgs &a, const SweepItemDev &it, bool up,
+                                             int part, Cx<double> *scrG) {
+  const GrainView &v = a.view;
+  const int lane = threadIdx.x;
+  const int cols = v.cols, gp = v.groups;
+  const int g = lane / cols;
+  const int c = lane - g * cols;
+  const int N1 = v.N1, Ne = v.Ne;
+  const size_t n1 = size_t(N1) * N1;
+  const double h = v.h;
+  const int k = it.angle;
+  const bool active = c < it.ncols && g < gp;
+  const unsigned x = unsigned(it.x0 + min(c, it.ncols - 1));
+  const int e0 = min(g, gp - 1) * EL;
+  const GlobalPtr<const int8_t> lab = global(v.labels + size_t(k) * n1);
+  const GlobalPtr<const double> F = global(v.fields + size_t(k - v.fieldBase) * n1);
+  const GlobalPtr<const double> rhoK = global(a.rho + size_t(k) * n1);
+  double *dbK = a.dbar + size_t(k) * n1 + x;
+  typedef double Pair __attribute__((ext_vector_type(2)));
+  const GlobalPtr<Pair> scr = global(reinterpret_cast<Pair *>(scrG));
+  // lanes past the energies and columns repeat others' with no weight
+  double ser[EL], res[EL];
+#pragma unroll
+  for (int j = 0; j < EL; ++j) {
+    const int e = min(e0 + j, Ne - 1);
+    ser[j] = -h * v.energy[e];
+    res[j] = active && e0 + j < Ne ? v.residue[e] : 0.0;
+  }
+  const int len = it.yhi - it.ylo + 1;
+  const int segs = (len + kGradSeg - 1) / kGradSeg;
+  const GlobalPtr<int> meta = global(reinterpret_cast<int *>(
+      scrG + size_t((a.maxLen + kGradSeg - 1) / kGradSeg) * (EL * 64)));
+  // the labels at which the recurrence enters the grain and leaves it
+  const int enter = up ? 2 : 3;
+  const size_t col = size_t(k) * N1 + x;
+  const int base = up ? v.idxInG[col] : v.idxInGt[col];
+  const size_t nIn = size_t(up ? v.nInG : v.nInGt) * Ne;
+  const GlobalPtr<const double> bIn = global(up ? v.bInG : v.bInGt);
+  const GlobalPtr<const double> dist = global(up ? v.distInG : v.distInGt);
+  const double sgn = up ? 1.0 : -1.0; // gamma~ steps with -conj(D)
+  auto rowOf = [&](int at) {
+    const int t = min(max(at, 0), len - 1);
+    return unsigned((up ? it.ylo + t : it.yhi - t) * N1) + x;
+  };
+  struct Row {
+    double re, im, es;
+  };
+  auto loadRow = [&](int at) {
+    const unsigned o = rowOf(at);
+    return Row{sgn * F[o], F[v.fieldPlane + o], F[2 * v.fieldPlane + o]};
+  };
+  // the step into a site: its parameters, the factor of the energies, the length
+  struct Step {
+    StepSite<double> p;
+    double f, hs;
+  };
+  // of a wavefront whose lanes are all inside the grain, past the first site
+  auto inner = [&](const Row &r0, const Row &r1) {
+    StepSite<double> p = stepSite(Cx<double>{(r0.re + r1.re) * 0.5, (r0.im + r1.im) * 0.5},
+                                  (r0.es + r1.es) * 0.5, h);
+    opaqueScalar(p.root);
+    return p;
+  };
+  auto general = [&](const Row &r0, const Row &r1, int l, int at, int ci) {
+    Step s;
+    s.f = at > 0 ? 1.0 : 0.5;
+    s.hs = h;
+    Cx<double> D = {(r0.re + r1.re) * 0.5, (r0.im + r1.im) * 0.5};
+    double es = (r0.es + r1.es) * 0.5;
+    if (at == 0) {
+      D = {0.5 * r1.re, 0.5 * r1.im};
+      es = 0.5 * r1.es;
+    }
+    if (l == enter) {
+      s.f = dist[ci];
+      s.hs = s.f * h;
+      D = {r1.re, r1.im};
+      es = r1.es;
+    }
+    s.p = stepSite(D, es, s.hs);
+    opaqueScalar(s.p.root);
+    return s;
+  };
+  // the state that a step starts from: the one before it or the in-value
+  auto origin = [&](Cx<double> y, int l, int ci, int j) {
+    if (l == enter) {
+      const size_t si = size_t(ci) * Ne + min(e0 + j, Ne - 1);
+      return Cx<double>{bIn[si], bIn[nIn + si]};
+    }
+    return y;
+  };
+
+  // forward: the states before the segments
+  int count = 0; // crossings into the grain so far
+  {
+    Cx<double> y[EL];
+#pragma unroll
+    for (int j = 0; j < EL; ++j) y[j] = {0.0, 0.0};
+    Row prev = {0.0, 0.0, 0.0}, row = loadRow(0);
+    int l = lab[rowOf(0)];
+    for (int sg = 0; sg < segs; ++sg) {
+#pragma unroll
+      for (int j = 0; j < EL; ++j) scr[size_t(sg * EL + j) * 64 + lane] = Pair{y[j].re, y[j].im};
+      int codes = count << 16;
+      for (int i = 0; i < kGradSeg; ++i) {
+        const int at = sg * kGradSeg + i;
+        if (at >= len) break;
+        codes |= l << (2 * i);
+        const Row next = loadRow(at + 1);
+        const int lNext = lab[rowOf(at + 1)];
+        if (at > 0 && __ballot(l != 1) == 0) {
+          const StepSite<double> p = inner(prev, row);
+#pragma unroll
+          for (int j = 0; j < EL; ++j) y[j] = stepEnergy(p, ser[j], y[j]);
+        } else {
+          const Step s = general(prev, row, l, at, base + count);
+#pragma unroll
+          for (int j = 0; j < EL; ++j) {
+            y[j] = stepEnergy(s.p, ser[j] * s.f, origin(y[j], l, base + count, j));
+            if (l == 0) y[j] = {0.0, 0.0};
+          }
+          if (l == enter) ++count;
+        }
+        prev = row;
+        row = next;
+        l = lNext;
+      }
+      meta[sg * 64 + lane] = codes;
+    }
+  }
+
+  // reverse: lam the adjoint that the step out of a site has left at it, half
+  // the same step's adjoint of D and the shift there
+  Cx<double> lam[EL];
+#pragma unroll
+  for (int j = 0; j < EL; ++j) lam[j] = {0.0, 0.0};
+  SiteBar half = {0.0, 0.0, 0.0};
+  double omega = 0.0;
+  for (int sg = segs - 1; sg >= 0; --sg) {
+    const int at0 = sg * kGradSeg;
+    Cx<double> y[kGradSeg + 1][EL];
+    Row row[kGradSeg + 1];
+#pragma unroll
+    for (int j = 0; j < EL; ++j) {
+      const Pair z = scr[size_t(sg * EL + j) * 64 + lane];
+      y[0][j] = {z.x, z.y};
+    }
+    const int codes = meta[sg * 64 + lane];
+#pragma unroll
+    for (int i = 0; i <= kGradSeg; ++i) row[i] = loadRow(at0 - 1 + i);
+    double rho[kGradSeg];
+#pragma unroll
+    for (int i = 0; i < kGradSeg; ++i) rho[i] = rhoK[rowOf(at0 + i)];
+    constexpr int kInner = 0x55555555 & ((1 << (2 * kGradSeg)) - 1);
+    const bool plain = at0 > 0 && __ballot((codes & 0xffff) != kInner) == 0;
+    int ci = base + (codes >> 16);
+#pragma unroll
+    for (int i = 0; i < kGradSeg; ++i) {
+      if (plain) {
+        const StepSite<double> p = inner(row[i], row[i + 1]);
+#pragma unroll
+        for (int j = 0; j < EL; ++j) y[i + 1][j] = stepEnergy(p, ser[j], y[i][j]);
+      } else {
+        const int l = codes >> (2 * i) & 3;
+        const Step s = general(row[i], row[i + 1], l, at0 + i, ci);
+#pragma unroll
+        for (int j = 0; j < EL; ++j) {
+          y[i + 1][j] = stepEnergy(s.p, ser[j] * s.f, origin(y[i][j], l, ci, j));
+          if (l == 0) y[i + 1][j] = {0.0, 0.0};
+        }
+        if (l == enter) ++ci;
+      }
+    }
+#pragma unroll
+    for (int i = kGradSeg - 1; i >= 0; --i) {
+      const int at = at0 + i;
+      if (at >= len) continue;
+      // (formed from the rows again, not kept from the steps)
+      opaque(row[i].re);
+      opaque(row[i].im);
+      opaque(row[i].es);
+      // the free-energy density, its own dependence on D and its adjoint of y
+      const double wr = rho[i] * row[i + 1].im, wi = -rho[i] * row[i + 1].re;
+      double su = 0.0, sw = 0.0;
+#pragma unroll
+      for (int j = 0; j < EL; ++j) {
+        su -= res[j] * y[i + 1][j].im;
+        sw += res[j] * y[i + 1][j].re;
+        lam[j].re += res[j] * wr;
+        lam[j].im += res[j] * wi;
+      }
+      // row.re is the recurrence's own (sgn times the field)
+      omega += rho[i] * (row[i + 1].re * su + row[i + 1].im * sw);
+      SiteBar bar = {half.re + rho[i] * su, half.im + rho[i] * sw, half.es};
+      AdjointSums sums;
+      if (plain) {
+        const StepSite<double> p = inner(row[i], row[i + 1]);
+#pragma unroll
+        for (int j = 0; j < EL; ++j)
+          lam[j] = stepAdjointSums(p, ser[j], y[i][j], y[i + 1][j], lam[j], sums);
+        const SiteBar d = sums.bar(h);
+        half = {0.5 * d.re, 0.5 * d.im, 0.5 * d.es};
+        addBar(bar, Cx<double>{half.re, half.im}, half.es);
+      } else {
+        const int l = codes >> (2 * i) & 3;
+        if (l == enter) --ci;
+        const Step s = general(row[i], row[i + 1], l, at, ci);
+        const bool step = l != 0, from = step && l != enter && at > 0;
+#pragma unroll
+        for (int j = 0; j < EL; ++j) {
+          const Cx<double> m = stepAdjointSums(s.p, ser[j] * s.f, origin(y[i][j], l, ci, j),
+                                               y[i + 1][j], lam[j], sums);
+          lam[j] = from ? m : Cx<double>{0.0, 0.0};
+        }
+        const SiteBar d = sums.bar(s.hs);
+        const double own = l == enter ? 1.0 : 0.5;
+        if (step) addBar(bar, Cx<double>{own * d.re, own * d.im}, own * d.es);
+        half = {0.0, 0.0, 0.0};
+        if (from) half = {0.5 * d.re, 0.5 * d.im, 0.5 * d.es};
+      }
+      const double re = groupSum(bar.re, gp, cols, c);
+      const double im = groupSum(bar.im, gp, cols, c);
+      const double es = groupSum(bar.es, gp, cols, c);
+      if (g == 0 && active) {
+        double *p = dbK + size_t(up ? it.ylo + at : it.yhi - at) * N1;
+        unsafeAtomicAdd(p, sgn * re);
+        unsafeAtomicAdd(p + a.framePlane, im);
+        unsafeAtomicAdd(p + 2 * a.framePlane, es);
+      }
+    }
+  }
+  // this item's share of the free-energy sum, stored by every lane alike (no
+  // branch on the lane index beside the fetch of the next item)
+  for (int m = 1; m < 64; m <<= 1) omega += __shfl_xor(omega, m);
+  a.partial[part] = omega;
+}
+
+// One wavefront per recurrence of an item.
+template <int EL>
+__global__ __launch_bounds__(64, kGradWaves) void gradientKernel(AdjointArgs a) {
+  Cx<double> *scr = a.scratch + size_t(blockIdx.x) * a.slotStride;
+  for (;;) {
+    // the branch-free fetch of adjointKernel
+    const int n =
+        __builtin_amdgcn_readfirstlane(atomicAdd(a.counter, threadIdx.x == 0 ? 1 : 0));
+    if (n >= 2 * a.numItems) break;
+    gradientItem<EL>(a, a.items[n >> 1], n & 1, n, scr);
+  }
+}
+
+template <int EL>
 __global__ __launch_bounds__(64, 2) void adjointKernel(AdjointArgs a) {
   Cx<double> *scrT = a.scratch + size_t(blockIdx.x) * 2 * a.slotStride;
   Cx<double> *scrG = scrT + a.slotStride;
@@ -814,7 +1086,7 @@ __global__ __launch_bounds__(64, 2) void adjointKernel(AdjointArgs a) {
     const int item =
         __builtin_amdgcn_readfirstlane(atomicAdd(a.counter, threadIdx.x == 0 ? 1 : 0));
     if (item >= a.numItems) break;
-    adjointItem<EL, RES>(a, a.items[item], item, scrT, scrG);
+    adjointItem<EL>(a, a.items[item], scrT, scrG);
   }
 }
 
@@ -1233,8 +1505,9 @@ void Grain::prepareAdjoint() {
     int dev = 0, cus = 0;
     SC_HIP(hipGetDevice(&dev));
     SC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    adjSlots_ = std::max(1, std::min(adjNumItems_, kAdjSlotsPerCU * std::max(cus, 1)));
-    dAdjPartial_ = devAlloc<double>(size_t(std::max(adjNumItems_, 1)));
+    adjSimds_ = 4 * std::max(cus, 1);
+    adjSlots_ = std::max(1, std::min(adjNumItems_, kAdjWaves * adjSimds_));
+    dAdjPartial_ = devAlloc<double>(2 * size_t(std::max(adjNumItems_, 1)));
     dAdjRho_ = devAlloc<double>(size_t(framePlane));
     dAdjDbar_ = devAlloc<double>(3 * size_t(framePlane));
     dAdjExt_ = devAlloc<double>(size_t(2 * s.Nc) * n0);
@@ -1242,9 +1515,13 @@ void Grain::prepareAdjoint() {
     dAdjGradA_ = devAlloc<double>(2 * n0);
     dAdjPart_ = devAlloc<double>(size_t(kFieldChunks) * size_t(2 * s.Nc + 2) * n0);
   }
-  // the slots' scratch for the setting of the checkpoints: every site
-  // (two buffers of maxLen sites), or segments of K sites (two buffers of
-  // ceil(maxLen / K) checkpoints and one segment each)
+}
+
+// The slots' scratch of the residual's reverse sweep for the setting of the
+// checkpoints: every site (two buffers of maxLen sites), or segments of K sites
+// (two buffers of ceil(maxLen / K) checkpoints and one segment each).
+void Grain::prepareReverse() {
+  prepareAdjoint();
   int K = 0;
   if (adjCk_ > 0) K = std::min(adjCk_, std::max(adjMaxLen_, 1));
   if (adjCk_ < 0) K = std::max(1, int(std::ceil(std::sqrt(double(std::max(adjMaxLen_, 1))))));
@@ -1284,6 +1561,10 @@ double Grain::freeEnergyGradient(double *grad, double *gradA) {
   ensureBoundaryInit();
   extendDelta();
   prepareAdjoint();
+  const int gradSlots =
+      std::max(1, std::min(2 * adjNumItems_, kGradWaves * adjSimds_));
+  if (!dGradScratch_)
+    dGradScratch_ = devAlloc<double>(size_t(gradSlots) * 2 * size_t(gradientStride(adjMaxLen_)));
   // A enters through the Doppler shift only with a penetration depth
   const bool withA = gradA != nullptr && s.lambda > 0.0;
   // (the seed of the free-energy density depends on the grain's geometry,
@@ -1317,10 +1598,10 @@ double Grain::freeEnergyGradient(double *grad, double *gradA) {
   a.items = reinterpret_cast<const SweepItemDev *>(adjItems_);
   a.numItems = adjNumItems_;
   a.counter = dCounter_;
-  a.scratch = reinterpret_cast<Cx<double> *>(dAdjScratch_);
-  a.slotStride = adjSlotStride_;
-  a.ck = adjCkUsed_;
-  a.ckSeg = adjCkSeg_;
+  a.scratch = reinterpret_cast<Cx<double> *>(dGradScratch_);
+  a.slotStride = gradientStride(adjMaxLen_);
+  a.ck = a.ckSeg = 0;
+  a.maxLen = adjMaxLen_;
   a.rho = dAdjRho_;
   a.seed = nullptr;
   a.dbar = dAdjDbar_;
@@ -1328,7 +1609,7 @@ double Grain::freeEnergyGradient(double *grad, double *gradA) {
   a.partial = dAdjPartial_;
   adjointResetCounter<<<1, 1, 0, stream_>>>(dCounter_);
   if (adjNumItems_ > 0) {
-    adjointKernel<kAdjEL, false><<<adjSlots_, 64, 0, stream_>>>(a);
+    gradientKernel<kAdjEL><<<gradSlots, 64, 0, stream_>>>(a);
     SC_HIP(hipGetLastError());
   }
   // 3. the rotation, basis and extension of the order parameter
@@ -1361,7 +1642,7 @@ double Grain::freeEnergyGradient(double *grad, double *gradA) {
   SC_HIP(hipGetLastError());
   // the free energy: the sweep's share from the items, the explicit terms
   clearReductions();
-  const int hSweep = queueSum(dAdjPartial_, nullptr, nullptr, adjNumItems_, 0);
+  const int hSweep = queueSum(dAdjPartial_, nullptr, nullptr, 2 * adjNumItems_, 0);
   std::vector<int> hSq;
   int hCurl = -1;
   queueExplicitFreeEnergy(hSq, hCurl);
@@ -1390,7 +1671,7 @@ double Grain::residualGradient(double *grad, double *gradA) {
   const bool doA = s.cfg.computeCurrent && s.lambda > 0.0;
   const bool withA = gradA != nullptr && doA;
   const size_t nd = size_t(2 * s.Nc) * n0;
-  prepareAdjoint();
+  prepareReverse();
   // the state the forward map overwrites: G's order parameter and vector
   // potential, the current, the energy density and the boundary out-values
   const size_t nNew = nd + 2 * n0;
@@ -1488,7 +1769,7 @@ double Grain::residualGradient(double *grad, double *gradA) {
   a.partial = dAdjPartial_;
   adjointResetCounter<<<1, 1, 0, stream_>>>(dCounter_);
   if (adjNumItems_ > 0) {
-    adjointKernel<kAdjEL, true><<<adjSlots_, 64, 0, stream_>>>(a);
+    adjointKernel<kAdjEL><<<adjSlots_, 64, 0, stream_>>>(a);
     SC_HIP(hipGetLastError());
   }
   // 5. the transposes of the site fields and of the order parameter's

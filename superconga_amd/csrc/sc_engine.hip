@@ -105,6 +105,7 @@ Grain::~Grain() {
   devFree(dWork2_);
   if (adjItems_) (void)hipFree(adjItems_);
   devFree(dAdjScratch_);
+  devFree(dGradScratch_);
   devFree(dAdjPartial_);
   devFree(dAdjRho_);
   devFree(dAdjDbar_);

@@ -412,8 +412,8 @@ private:
   // the free-energy gradient (sc_adjoint.hip)
   void queueExplicitFreeEnergy(std::vector<int> &hSq, int &hCurl);
   void *adjItems_ = nullptr;
-  int adjNumItems_ = 0, adjMaxLen_ = 0, adjSlots_ = 0;
-  double *dAdjScratch_ = nullptr, *dAdjPartial_ = nullptr, *dAdjRho_ = nullptr,
+  int adjNumItems_ = 0, adjMaxLen_ = 0, adjSimds_ = 0, adjSlots_ = 0;
+  double *dAdjScratch_ = nullptr, *dGradScratch_ = nullptr, *dAdjPartial_ = nullptr, *dAdjRho_ = nullptr,
          *dAdjDbar_ = nullptr, *dAdjExt_ = nullptr, *dAdjGrad_ = nullptr,
          *dAdjGradA_ = nullptr, *dAdjPart_ = nullptr;
   // the residual gradient's buffers: rD, rA, the Poisson seed and its
@@ -423,6 +423,7 @@ private:
          *dResJbar_ = nullptr, *dResZero_ = nullptr, *dResMean_ = nullptr, *dResSeed_ = nullptr,
          *dResSave_ = nullptr;
   void prepareAdjoint();
+  void prepareReverse();
   int adjCk_ = -1, adjCkUsed_ = 0, adjCkSeg_ = 0;
   bool adjRhoReady_ = false; // dAdjRho_ holds the free-energy seed
   int nkRestarts_ = 4;
