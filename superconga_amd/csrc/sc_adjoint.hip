@@ -221,26 +221,90 @@ __device__ __forceinline__ void gatherFrame(const double *const *planes, int nPl
     }
 }
 
+// The same for a tile of kTapTile x kTapTile sites, one to a thread: the frame
+// sites that may tap them lie in a box of at most 15 sqrt(2) + 4 sites a side
+// (and one more on either side for the rounding of its corners).  Their taps,
+// weights and values are formed once, in LDS, where every site by itself forms
+// those of its 16 and waits for each site's values in turn: a square of 606
+// sites a side, 128 angles: 14.4 ms before, 2.1 with it.  The sums are taken
+// in the same order.
+constexpr int kTapTile = 16, kTapBox = 28;
+struct TapLds {
+  int tap[kTapBox * kTapBox]; // Yi << 16 | Xi, negative: none
+  double fx[kTapBox * kTapBox], fy[kTapBox * kTapBox], val[2][kTapBox * kTapBox];
+};
+template <int P>
+__device__ __forceinline__ void gatherTile(const double *const (&planes)[P], bool own, int px,
+                                           int py, int N0, int N1, double c, double s, TapLds &lds,
+                                           double (&acc)[3]) {
+  const double sh = 0.5 * double(N0 - 1), h1 = 0.5 * double(N1 - 1);
+  // the box, from the tile's corners
+  const int tx = px - int(threadIdx.x % kTapTile), ty = py - int(threadIdx.x / kTapTile);
+  const double X0 = double(tx) - sh, Y0 = double(ty) - sh, w = double(kTapTile - 1);
+  const double xc = X0 * c + Y0 * s + h1, yc = -X0 * s + Y0 * c + h1;
+  const int bx0 = max(int(floor(xc + fmin(w * c, 0.0) + fmin(w * s, 0.0))) - 2, 0);
+  const int by0 = max(int(floor(yc + fmin(-w * s, 0.0) + fmin(w * c, 0.0))) - 2, 0);
+  const int bx1 = min(int(floor(xc + fmax(w * c, 0.0) + fmax(w * s, 0.0))) + 3, N1 - 1);
+  const int by1 = min(int(floor(yc + fmax(-w * s, 0.0) + fmax(w * c, 0.0))) + 3, N1 - 1);
+  const int bw = min(max(bx1 - bx0 + 1, 0), kTapBox), bh = min(max(by1 - by0 + 1, 0), kTapBox);
+  __syncthreads(); // the last frame's are read
+  for (int i = threadIdx.x; i < bw * bh; i += kTapTile * kTapTile) {
+    const int y = i / bw, x = i - y * bw;
+    const size_t fi = size_t(by0 + y) * N1 + bx0 + x;
+    const int at = y * kTapBox + x;
+#pragma unroll
+    for (int q = 0; q < P; ++q) lds.val[q][at] = planes[q][fi];
+    const RotSample r = rotatedCell(bx0 + x, by0 + y, N1, N0, c, s);
+    const int Yi = r.idx / N0, Xi = r.idx - Yi * N0;
+    lds.tap[at] = r.valid ? Yi << 16 | Xi : -1;
+    lds.fx[at] = r.fx;
+    lds.fy[at] = r.fy;
+  }
+  __syncthreads();
+  if (!own) return;
+  const double Pcx = double(px) - sh, Pcy = double(py) - sh;
+  const double xf = Pcx * c + Pcy * s + h1, yf = -Pcx * s + Pcy * c + h1;
+  const int xi = int(floor(xf)) - 1, yi = int(floor(yf)) - 1;
+  const int x0 = max(xi, bx0), x1 = min(xi + 3, bx0 + bw - 1);
+  const int y0 = max(yi, by0), y1 = min(yi + 3, by0 + bh - 1);
+  for (int cy = y0; cy <= y1; ++cy)
+    for (int cx = x0; cx <= x1; ++cx) {
+      const int at = (cy - by0) * kTapBox + cx - bx0;
+      const int tap = lds.tap[at];
+      const int dx = px - (tap & 0xffff), dy = py - (tap >> 16);
+      if (tap < 0 || dx < 0 || dx > 1 || dy < 0 || dy > 1) continue;
+      const double fx = lds.fx[at], fy = lds.fy[at];
+      const double wt = (dy ? fy : 1.0 - fy) * (dx ? fx : 1.0 - fx);
+#pragma unroll
+      for (int q = 0; q < P; ++q) acc[q] += lds.val[q][at] * wt;
+    }
+}
+
 // The frames are split into kFieldChunks ranges (blockIdx.y), each thread
 // summing its range into its own slot of part ([chunk][plane][site], planes
 // Re/Im of every component, then A_x and A_y): many more threads to hide
 // the loads' latency, and fieldsAdjointSumKernel adds the ranges in order.
+// Sites at the grid's lower edges take their wider window one by one.
 constexpr int kFieldChunks = 8;
-__global__ void fieldsAdjointKernel(GrainView v, const double *dbar, long long framePlane,
-                                    bool withA, double *part) {
-  const long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(kTapTile *kTapTile) void fieldsAdjointKernel(
+    GrainView v, const double *dbar, long long framePlane, bool withA, double *part) {
+  __shared__ TapLds lds;
   const int N0 = v.N0, N1 = v.N1, Na = v.Na, Nc = v.Nc;
   const size_t n0 = size_t(N0) * N0, n1 = size_t(N1) * N1;
-  if (p >= (long long)n0) return;
-  const int px = int(p % N0), py = int(p / N0);
+  const int tiles = (N0 + kTapTile - 1) / kTapTile;
+  const int px = int(blockIdx.x) % tiles * kTapTile + int(threadIdx.x) % kTapTile;
+  const int py = int(blockIdx.x) / tiles * kTapTile + int(threadIdx.x) / kTapTile;
+  const bool in = px < N0 && py < N0, edge = px <= 1 || py <= 1;
   const int chunk = blockIdx.y;
   const int k0 = chunk * Na / kFieldChunks, k1 = (chunk + 1) * Na / kFieldChunks;
   double dr[4] = {0, 0, 0, 0}, di[4] = {0, 0, 0, 0};
   double ax = 0.0, ay = 0.0;
   for (int k = k0; k < k1; ++k) {
     const double *pl[2] = {dbar + size_t(k) * n1, dbar + framePlane + size_t(k) * n1};
+    const double oc = double(v.opCos[k]), os = double(v.opSin[k]);
     double acc[3] = {0.0, 0.0, 0.0};
-    gatherFrame(pl, 2, px, py, N0, N1, double(v.opCos[k]), double(v.opSin[k]), acc);
+    gatherTile<2>(pl, in && !edge, px, py, N0, N1, oc, os, lds, acc);
+    if (in && edge) gatherFrame(pl, 2, px, py, N0, N1, oc, os, acc);
     if (acc[0] != 0.0 || acc[1] != 0.0) {
       for (int c = 0; c < Nc && c < 4; ++c) {
         const double b = v.basis[c * Na + k];
@@ -250,12 +314,16 @@ __global__ void fieldsAdjointKernel(GrainView v, const double *dbar, long long f
     }
     if (withA) {
       const double *pe[1] = {dbar + 2 * framePlane + size_t(k) * n1};
+      const double ac = double(v.aCos[k]), as = double(v.aSin[k]);
       double ae[3] = {0.0, 0.0, 0.0};
-      gatherFrame(pe, 1, px, py, N0, N1, double(v.aCos[k]), double(v.aSin[k]), ae);
+      gatherTile<1>(pe, in && !edge, px, py, N0, N1, ac, as, lds, ae);
+      if (in && edge) gatherFrame(pe, 1, px, py, N0, N1, ac, as, ae);
       ax += double(v.charge) * v.vFx[k] * ae[0];
       ay += double(v.charge) * v.vFy[k] * ae[0];
     }
   }
+  if (!in) return;
+  const size_t p = size_t(py) * N0 + px;
   const int planes = 2 * Nc + 2;
   double *out = part + size_t(chunk) * planes * n0 + p;
   for (int c = 0; c < Nc && c < 4; ++c) {
@@ -264,6 +332,11 @@ __global__ void fieldsAdjointKernel(GrainView v, const double *dbar, long long f
   }
   out[size_t(2 * Nc) * n0] = ax;
   out[size_t(2 * Nc + 1) * n0] = ay;
+}
+
+unsigned tapTiles(int N0) {
+  const unsigned t = unsigned((N0 + kTapTile - 1) / kTapTile);
+  return t * t;
 }
 
 // The frame ranges added in order: extBar (Re/Im of every component, the
@@ -1613,7 +1686,7 @@ double Grain::freeEnergyGradient(double *grad, double *gradA) {
     SC_HIP(hipGetLastError());
   }
   // 3. the rotation, basis and extension of the order parameter
-  fieldsAdjointKernel<<<dim3(blocksFor(static_cast<long long>(n0)), kFieldChunks), 256, 0,
+  fieldsAdjointKernel<<<dim3(tapTiles(s.N0), kFieldChunks), kTapTile * kTapTile, 0,
                         stream_>>>(v, dAdjDbar_, framePlane, withA, dAdjPart_);
   SC_HIP(hipGetLastError());
   fieldsAdjointSumKernel<<<blocksFor(static_cast<long long>(2 * s.Nc + 2) * n0), 256, 0,
@@ -1774,7 +1847,7 @@ double Grain::residualGradient(double *grad, double *gradA) {
   }
   // 5. the transposes of the site fields and of the order parameter's
   // extension, then the identity part
-  fieldsAdjointKernel<<<dim3(blocksFor(static_cast<long long>(n0)), kFieldChunks), 256, 0,
+  fieldsAdjointKernel<<<dim3(tapTiles(s.N0), kFieldChunks), kTapTile * kTapTile, 0,
                         stream_>>>(v, dAdjDbar_, framePlane, withA, dAdjPart_);
   SC_HIP(hipGetLastError());
   fieldsAdjointSumKernel<<<blocksFor(static_cast<long long>(2 * s.Nc + 2) * n0), 256, 0,
