@@ -885,10 +885,12 @@ __device__ void adjointItem(const AdjointArgs &a, const SweepItemDev &it, Cx<dou
 // and reading a state 32 bytes.  One wavefront that went down, up and down again,
 // with checkpoints every sqrt(length) sites and the segments in the scratch, took
 // some 300 instructions and 64 bytes per site and energy of both recurrences in
-// one chain of three passes; this takes 2 (49 + 49 + 40) and 2 * 32 / kGradSeg
+// one chain of three passes; this takes 2 (49 + 37 + 40) and 2 * 32 / kGradSeg
 // in two independent chains of two.  A square of 606 sites a side, 12 energies,
-// 128 angles: 19.0 ms before, 11.4 with it.  Segments of 6 sites need 57 registers
-// more than the 256 of two wavefronts a SIMD.
+// 128 angles: 19.0 ms before, 10.6 with it (the forward pass 4.2).  Segments of
+// 2 and 3 sites, of fewer instructions and more bytes, take 11.6 and 11.3 ms; 6
+// need 57 registers more than the 256 of two wavefronts a SIMD; the loads of a
+// segment issued a segment ahead gain nothing.
 constexpr int kGradSeg = 4;   // sites of a segment
 constexpr int kGradWaves = 2; // wavefronts per SIMD
 // complex elements of a slot's scratch
@@ -992,15 +994,16 @@ __device__ __forceinline__ void gradientItem(const AdjointArgs &a, const SweepIt
 
   // forward: the states before the segments
   int count = 0; // crossings into the grain so far
+  Cx<double> y[kGradSeg + 1][EL];
   {
-    Cx<double> y[EL];
+    Cx<double>(&y0)[EL] = y[kGradSeg];
 #pragma unroll
-    for (int j = 0; j < EL; ++j) y[j] = {0.0, 0.0};
+    for (int j = 0; j < EL; ++j) y0[j] = {0.0, 0.0};
     Row prev = {0.0, 0.0, 0.0}, row = loadRow(0);
     int l = lab[rowOf(0)];
     for (int sg = 0; sg < segs; ++sg) {
 #pragma unroll
-      for (int j = 0; j < EL; ++j) scr[size_t(sg * EL + j) * 64 + lane] = Pair{y[j].re, y[j].im};
+      for (int j = 0; j < EL; ++j) scr[size_t(sg * EL + j) * 64 + lane] = Pair{y0[j].re, y0[j].im};
       int codes = count << 16;
       for (int i = 0; i < kGradSeg; ++i) {
         const int at = sg * kGradSeg + i;
@@ -1011,13 +1014,13 @@ __device__ __forceinline__ void gradientItem(const AdjointArgs &a, const SweepIt
         if (at > 0 && __ballot(l != 1) == 0) {
           const StepSite<double> p = inner(prev, row);
 #pragma unroll
-          for (int j = 0; j < EL; ++j) y[j] = stepEnergy(p, ser[j], y[j]);
+          for (int j = 0; j < EL; ++j) y0[j] = stepEnergy(p, ser[j], y0[j]);
         } else {
           const Step s = general(prev, row, l, at, base + count);
 #pragma unroll
           for (int j = 0; j < EL; ++j) {
-            y[j] = stepEnergy(s.p, ser[j] * s.f, origin(y[j], l, base + count, j));
-            if (l == 0) y[j] = {0.0, 0.0};
+            y0[j] = stepEnergy(s.p, ser[j] * s.f, origin(y0[j], l, base + count, j));
+            if (l == 0) y0[j] = {0.0, 0.0};
           }
           if (l == enter) ++count;
         }
@@ -1038,7 +1041,6 @@ __device__ __forceinline__ void gradientItem(const AdjointArgs &a, const SweepIt
   double omega = 0.0;
   for (int sg = segs - 1; sg >= 0; --sg) {
     const int at0 = sg * kGradSeg;
-    Cx<double> y[kGradSeg + 1][EL];
     Row row[kGradSeg + 1];
 #pragma unroll
     for (int j = 0; j < EL; ++j) {
@@ -1054,8 +1056,9 @@ __device__ __forceinline__ void gradientItem(const AdjointArgs &a, const SweepIt
     constexpr int kInner = 0x55555555 & ((1 << (2 * kGradSeg)) - 1);
     const bool plain = at0 > 0 && __ballot((codes & 0xffff) != kInner) == 0;
     int ci = base + (codes >> 16);
+    // (the last state is the one before the segment above, or the forward pass's)
 #pragma unroll
-    for (int i = 0; i < kGradSeg; ++i) {
+    for (int i = 0; i < kGradSeg - 1; ++i) {
       if (plain) {
         const StepSite<double> p = inner(row[i], row[i + 1]);
 #pragma unroll
@@ -1071,6 +1074,7 @@ __device__ __forceinline__ void gradientItem(const AdjointArgs &a, const SweepIt
         if (l == enter) ++ci;
       }
     }
+    if (!plain && (codes >> (2 * (kGradSeg - 1)) & 3) == enter) ++ci;
 #pragma unroll
     for (int i = kGradSeg - 1; i >= 0; --i) {
       const int at = at0 + i;
@@ -1128,6 +1132,8 @@ __device__ __forceinline__ void gradientItem(const AdjointArgs &a, const SweepIt
         unsafeAtomicAdd(p + 2 * a.framePlane, es);
       }
     }
+#pragma unroll
+    for (int j = 0; j < EL; ++j) y[kGradSeg][j] = y[0][j];
   }
   // this item's share of the free-energy sum, stored by every lane alike (no
   // branch on the lane index beside the fetch of the next item)
