@@ -1829,6 +1829,10 @@ void Grain::jacobianVector(const double *dv, double *djv, bool inValues, bool sc
     dTanOutG_ = devAlloc<double>(std::max<size_t>(1, size_t(2 * s.nOutG * s.Ne)));
     dTanOutGt_ = devAlloc<double>(std::max<size_t>(1, size_t(2 * s.nOutGt * s.Ne)));
     dTanScratch_ = devAlloc<double>(size_t(adjSlots_) * 4 * size_t(adjMaxLen_) * kAdjointEL * 64);
+    // every product writes the same sites (the field tiles; the inside sites and
+    // the extension's targets): the others stay zero
+    SC_HIP(hipMemsetAsync(dTanFields_, 0, 3 * size_t(framePlane) * sizeof(double), stream_));
+    SC_HIP(hipMemsetAsync(dTanG_, 0, 4 * size_t(framePlane) * sizeof(double), stream_));
   }
   // the state's fields, then the tangents of the extended order parameter
   // and of the site fields (the induced vector potential's share of the
@@ -1849,7 +1853,6 @@ void Grain::jacobianVector(const double *dv, double *djv, bool inValues, bool sc
   tv.fluxDensity = 0.0;
   tv.useInduced = doA ? 1 : 0;
   tv.useField = doA ? 1 : 0;
-  SC_HIP(hipMemsetAsync(dTanFields_, 0, 3 * size_t(framePlane) * sizeof(double), stream_));
   const int nt = s.fieldTileStart[size_t(s.Na)];
   if (nt > 0) {
     fieldsKernel<<<xcdGrid(nt), 256, 0, stream_>>>(tv, dFieldTiles_, nt, 0, framePlane,
@@ -1857,7 +1860,6 @@ void Grain::jacobianVector(const double *dv, double *djv, bool inValues, bool sc
     SC_HIP(hipGetLastError());
   }
   // the sweep's tangent
-  SC_HIP(hipMemsetAsync(dTanG_, 0, 4 * size_t(framePlane) * sizeof(double), stream_));
   tangentSweep(sweepView(kAdjointEL), dTanFields_, adjItems_, adjNumItems_, dCounter_,
                dTanScratch_, static_cast<long long>(adjMaxLen_) * kAdjointEL * 64,
                inValues ? dv + nx : nullptr, inValues ? dv + nx + nG : nullptr, dTanOutG_,
