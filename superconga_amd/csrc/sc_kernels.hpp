@@ -6,58 +6,87 @@
 
 namespace scamd {
 
-// Order parameter and Doppler shift at site (x, y) of frame k, from the
+// Order parameter and Doppler shift at sites (x, y[i]) of frame k, from the
 // extended order parameter and the vector potential on the N0 grid
 // (OrderParameter.h:232-269, RiccatiSolver.h:127-176,
 // VectorPotential_Kernel.h:21-99, Gauges.h:25-62).
-__device__ __forceinline__ void siteFields(const GrainView &v, int k, int x,
-                                           int y, double &dre, double &dim,
-                                           double &es) {
+template <int R>
+__device__ __forceinline__ void siteFieldRows(const GrainView &v, int k, int x, const int (&y)[R],
+                                              double (&dre)[R], double (&dim)[R],
+                                              double (&es)[R]) {
   const int N0 = v.N0, N1 = v.N1;
   const size_t n0 = size_t(N0) * N0;
-  dre = 0.0;
-  dim = 0.0;
-  const RotSample r =
-      rotatedCell(x, y, N1, N0, double(global(v.opCos)[k]), double(global(v.opSin)[k]));
-  if (r.valid) {
-    for (int c = 0; c < v.Nc; ++c) {
-      const double b = global(v.basis)[c * v.Na + k];
-      const double *p = v.extDelta + size_t(c) * 2 * n0;
-      dre += b * bilinear(p, N0, r);
-      dim += b * bilinear(p + n0, N0, r);
+  // (a site with no cell reads the first one: no branch, so that the loads of
+  // all rows are in flight together)
+  auto cells = [&](double c, double s, RotSample (&r)[R]) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      r[i] = rotatedCell(x, y[i], N1, N0, c, s);
+      r[i].idx = r[i].valid ? r[i].idx : 0;
+    }
+  };
+  RotSample r[R];
+  cells(double(global(v.opCos)[k]), double(global(v.opSin)[k]), r);
+#pragma unroll
+  for (int i = 0; i < R; ++i) dre[i] = dim[i] = es[i] = 0.0;
+  for (int c = 0; c < v.Nc; ++c) {
+    const double b = global(v.basis)[c * v.Na + k];
+    const double *p = v.extDelta + size_t(c) * 2 * n0;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const double re = bilinear(p, N0, r[i]), im = bilinear(p + n0, N0, r[i]);
+      if (r[i].valid) {
+        dre[i] += b * re;
+        dim[i] += b * im;
+      }
     }
   }
-  es = 0.0;
   if (v.useField) {
-    double ax = 0.0, ay = 0.0;
+    double ax[R], ay[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) ax[i] = ay[i] = 0.0;
     if (v.useInduced) {
-      const RotSample q =
-          rotatedCell(x, y, N1, N0, double(global(v.aCos)[k]), double(global(v.aSin)[k]));
-      if (q.valid) {
-        ax = bilinear(v.A, N0, q) * v.lambdaInv2;
-        ay = bilinear(v.A + n0, N0, q) * v.lambdaInv2;
+      cells(double(global(v.aCos)[k]), double(global(v.aSin)[k]), r);
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const double a0 = bilinear(v.A, N0, r[i]), a1 = bilinear(v.A + n0, N0, r[i]);
+        ax[i] = r[i].valid ? a0 * v.lambdaInv2 : 0.0;
+        ay[i] = r[i].valid ? a1 * v.lambdaInv2 : 0.0;
       }
     }
     const double off = -0.5 * double(N1 - 1);
-    const double px0 = (double(x) + off) * v.h, py0 = (double(y) + off) * v.h;
     const double c = global(v.saCos)[k], s = global(v.saSin)[k];
-    const double px = px0 * c - py0 * s, py = px0 * s + py0 * c;
-    double ex, ey;
-    if (v.gauge == 0) {
-      ex = 0.0;
-      ey = px * v.fluxDensity;
-    } else if (v.gauge == 1) {
-      const double f = 0.5 * v.fluxDensity;
-      ex = -py * f;
-      ey = px * f;
-    } else {
-      const double r2 = fmax(px * px + py * py, 1e-7);
-      const double f = v.fluxDensity * v.area / (2.0 * M_PI * r2);
-      ex = -py * f;
-      ey = px * f;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const double px0 = (double(x) + off) * v.h, py0 = (double(y[i]) + off) * v.h;
+      const double px = px0 * c - py0 * s, py = px0 * s + py0 * c;
+      double ex, ey;
+      if (v.gauge == 0) {
+        ex = 0.0;
+        ey = px * v.fluxDensity;
+      } else if (v.gauge == 1) {
+        const double f = 0.5 * v.fluxDensity;
+        ex = -py * f;
+        ey = px * f;
+      } else {
+        const double r2 = fmax(px * px + py * py, 1e-7);
+        const double f = v.fluxDensity * v.area / (2.0 * M_PI * r2);
+        ex = -py * f;
+        ey = px * f;
+      }
+      es[i] = double(v.charge) *
+              (global(v.vFx)[k] * (ax[i] + ex) + global(v.vFy)[k] * (ay[i] + ey));
     }
-    es = double(v.charge) * (global(v.vFx)[k] * (ax + ex) + global(v.vFy)[k] * (ay + ey));
   }
+}
+__device__ __forceinline__ void siteFields(const GrainView &v, int k, int x, int y, double &dre,
+                                           double &dim, double &es) {
+  const int ys[1] = {y};
+  double re[1], im[1], e[1];
+  siteFieldRows<1>(v, k, x, ys, re, im, e);
+  dre = re[0];
+  dim = im[0];
+  es = e[0];
 }
 
 // The sweep's work counters (sc_view.hpp).
@@ -72,6 +101,10 @@ __global__ void resetCounter(int *c) {
 // sweep may read there), 16 columns x 16 rows per pass, so that the writes
 // of a row of the tile are contiguous.  F is planar [3][frames][N1^2] with
 // plane stride `plane`; frame k is at (k - k0) * N1^2.
+// A thread takes two of its rows at a time: their taps wait for memory together
+// (octagon of 930 sites a side, 128 angles: 1.69 ms one by one, 1.42 by two, 1.51
+// by four, which spill).
+constexpr int kFieldRows = 2;
 __device__ __forceinline__ void fieldsTile(const GrainView &v, const int *tl, int k0,
                                            long long plane, double *Fout) {
   const GlobalPtr<const int> tg = global(tl);
@@ -80,13 +113,20 @@ __device__ __forceinline__ void fieldsTile(const GrainView &v, const int *tl, in
   const int N1 = v.N1;
   if (x >= N1) return;
   const size_t base = size_t(k - k0) * N1 * N1 + x;
-  for (int y = y0 + int(threadIdx.x >> 4); y <= y1; y += 16) {
-    double re, im, es;
-    siteFields(v, k, x, y, re, im, es);
-    const size_t i = base + size_t(y) * N1;
-    F[i] = re;
-    F[plane + i] = im;
-    F[2 * plane + i] = es;
+  for (int y = y0 + int(threadIdx.x >> 4); y <= y1; y += 16 * kFieldRows) {
+    int ys[kFieldRows];
+    double re[kFieldRows], im[kFieldRows], es[kFieldRows];
+#pragma unroll
+    for (int i = 0; i < kFieldRows; ++i) ys[i] = min(y + 16 * i, y1);
+    siteFieldRows<kFieldRows>(v, k, x, ys, re, im, es);
+#pragma unroll
+    for (int i = 0; i < kFieldRows; ++i) {
+      if (y + 16 * i > y1) break;
+      const size_t at = base + size_t(ys[i]) * N1;
+      F[at] = re[i];
+      F[plane + at] = im[i];
+      F[2 * plane + at] = es[i];
+    }
   }
 }
 __global__ void fieldsKernel(GrainView v, const int *tiles, int numTiles, int k0,

@@ -32,7 +32,7 @@ namespace scamd {
 // in increasing order; the first chunk starts the sums.  WIDE: two neighbouring
 // energies per thread (Ne even), which share the rotation and read each tap in
 // one 16-byte load: by one energy a thread the rotations alone were 2.2 of the
-// 4.65 ms of 720 angles, 32 energies and 70000 sites; FIGURE ms with two.
+// 4.65 ms of 720 angles, 32 energies and 70000 sites; 3.64 ms with two.
 template <bool WIDE>
 __global__ void ldosGatherKernel(GrainView v, const int *sites, int numSites, int k0, int k1,
                                  int first, double *acc) {
