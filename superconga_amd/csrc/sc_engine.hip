@@ -1246,7 +1246,7 @@ void Grain::solveVectorPotential(const double *dj, double *dout) {
     sumKernel<<<blocks, 256, 0, stream_>>>(dj + size_t(d) * n0, nullptr, nullptr,
                                            static_cast<long long>(n0), 0, part);
     SC_HIP(hipGetLastError());
-    finishMeanKernel<<<1, 1, 0, stream_>>>(part, blocks, static_cast<double>(s.numGrain),
+    finishMeanKernel<<<1, 256, 0, stream_>>>(part, blocks, static_cast<double>(s.numGrain),
                                            dMean_ + d);
     SC_HIP(hipGetLastError());
   }

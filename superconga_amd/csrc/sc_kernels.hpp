@@ -515,12 +515,24 @@ __global__ void combineTermsKernel(double *y, const double *base, double a, Comb
   for (int q = 0; q < m; ++q) acc += t.c[q] * t.v[q][i];
   y[i] = acc;
 }
-// mean = (sum of the block partials, in block order) / count
-__global__ void finishMeanKernel(const double *partials, long long blocks, double count,
-                                 double *mean) {
+// mean = (sum of the block partials, in block order) / count: one block loads
+// them side by side and one thread adds them from LDS (loaded one by one, each
+// waiting for memory, 1024 partials took 56 us; 9 us so).
+__global__ __launch_bounds__(256) void finishMeanKernel(const double *partials, long long blocks,
+                                                        double count, double *mean) {
+  __shared__ double sh[1024];
   double s = 0.0;
-  for (long long b = 0; b < blocks; ++b) s += partials[b];
-  *mean = s / count;
+  for (long long b0 = 0; b0 < blocks; b0 += 1024) {
+    const int n = int(blocks - b0 < 1024 ? blocks - b0 : 1024);
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += 256) sh[i] = partials[b0 + i];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll 16
+      for (int i = 0; i < n; ++i) s += sh[i];
+    }
+  }
+  if (threadIdx.x == 0) *mean = s / count;
 }
 
 // Dot products of one vector with up to kMaxDots others in one pass over it:
