@@ -254,8 +254,9 @@ int sc_residual_gradient(sc_context *ctx, double *grad, double *grad_a, double *
  * reference. */
 int sc_jacobian_vector(sc_context *ctx, const double *v, double *jv);
 
-/* How the reverse sweeps of sc_free_energy_gradient(_ex) and
- * sc_residual_gradient keep the coherence functions they run back over:
+/* How the reverse sweep of sc_residual_gradient keeps the coherence
+ * functions it runs back over (that of sc_free_energy_gradient(_ex) keeps
+ * every fourth site whatever k, and takes those in between again):
  * k > 0 keeps a checkpoint every k sites and integrates each segment again
  * when the reverse passes reach it (twice the forward steps, scratch of
  * ceil(L / k) checkpoints and one segment instead of L sites for the

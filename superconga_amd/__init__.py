@@ -390,7 +390,7 @@ class Simulation:
                                            int(bool(fp64_fallback)), int(bool(fix_phase))))
 
     def set_adjoint_checkpoints(self, k):
-        """The reverse sweeps' storage: k > 0 a checkpoint every k sites
+        """The residual's reverse sweep's storage: k > 0 a checkpoint every k sites
         (each segment integrated again), -1 (the default) picks
         k = ceil(sqrt(longest trajectory)), 0 keeps every site.  The
         gradients are the same."""

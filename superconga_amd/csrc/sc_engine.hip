@@ -301,8 +301,8 @@ bool sweepVariantExists(int el, int waves, bool keldysh) {
 // 15.2 against 12.7 in FP32).
 SweepShape defaultSweepShape(const std::vector<const Setup *> &grains, int precision) {
   const bool dp = precision == PREC_FP64;
-  const double latency = 3.0, latencyPer = dp ? 1.2 : 0.2, issue = dp ? 1.6 : 0.2;
-  const double shared = dp ? 0.6 : 1.5, sharedLess = dp ? 0.2 : 1.0;
+  const double latency = 3.0, latencyPer = dp ? 1.2 : 0.3, issue = dp ? 1.6 : 0.2;
+  const double shared = dp ? 0.6 : 3.0, sharedLess = dp ? 0.2 : 2.0;
   // compiled without register spills (or nearly: 3 at three wavefronts)
   const SweepShape fp64[] = {{1, 4, 16}, {3, 3, 16}, {4, 2, 16}, {5, 2, 16}, {6, 2, 16}, {7, 2, 8},
                              {8, 2, 8}};

@@ -214,7 +214,7 @@ public:
   // The same on host vectors [Delta planes (Nc x 2 x N0^2), A planes
   // (2 x N0^2, in the setters' units)], in-values held fixed, unscreened.
   void jacobianVectorHost(const double *v, double *jv);
-  // The reverse sweeps' storage of the coherence functions: 0 keeps every
+  // The residual's reverse sweep's storage of the coherence functions: 0 keeps every
   // site, k > 0 keeps checkpoints every k sites and integrates each segment
   // again when the reverse passes reach it, -1 (the default) picks
   // k = ceil(sqrt(longest trajectory)).  Results are the same either way.
